@@ -39,6 +39,7 @@ SOURCES = [
     "rotary.hip",
     "causal_conv1d.hip",
     "gemv.hip",
+    "gemv_batch.hip",
     "flash_attention.hip",
     "fa_noalloc.hip",
 ]
@@ -66,10 +67,10 @@ EXTRA_FLAGS = {
 # The count is right only if those loads stay between the copies and the
 # wait, which the compiler does not promise for loads of read-only memory,
 # so the device assembly of these sources is checked on every build.
-# flash_attention.hip waits for its copies by counting only younger copies
-# (inline assembly, which the compiler keeps in order), so only its use of M0
-# is checked there.
-COPY_WAIT_CHECKED = {"gemv.hip": True, "flash_attention.hip": False}
+# flash_attention.hip and gemv_batch.hip wait for their copies by counting only
+# younger copies (inline assembly, which the compiler keeps in order), so only
+# their use of M0 is checked.
+COPY_WAIT_CHECKED = {"gemv.hip": True, "gemv_batch.hip": False, "flash_attention.hip": False}
 
 
 def check_copy_waits(asm_text, src="", waits=True):
