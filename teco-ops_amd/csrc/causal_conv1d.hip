@@ -17,7 +17,8 @@
 //   token stride 1 (e.g. [batch, dim, seqlen], the reference's [dim, tokens]):
 //     a wave streams whole rows, lanes on consecutive 8-token chunks ->
 //     16-byte loads / stores, the W-1 overlap passed between lanes in
-//     registers (conv1d_rows_kernel);
+//     registers (conv1d_rows_kernel); a varlen batch's channel is streamed
+//     across its sequences (conv1d_axis_kernel);
 //   channel stride 1 with dim % 8 == 0 (the reference C layout [tokens, dim]):
 //     a lane owns 8 consecutive channels (one 16-byte vector per token) of a
 //     16-token chunk of the global token axis; the W-1 rows before the chunk
@@ -25,7 +26,8 @@
 //   otherwise: consecutive lanes take consecutive channels of one 16-token
 //     chunk with 2-byte accesses (conv1d_kernel).
 // Only one lane of a (sequence, channel) touches conv_state, reading the old
-// state before writing the new one, so there is no cross-lane race.
+// state before writing the new one, so there is no cross-lane race
+// (conv1d_axis_kernel: one workgroup, with a barrier between the two).
 // HBM-bound: algorithmic bytes = 2 * (x + out) + weights + bias + state.
 #include "common.h"
 #include "device.h"
@@ -165,152 +167,366 @@ __device__ __forceinline__ void conv1d_body(const ConvArgs &a, int b, int d, int
     }
 }
 
+// A row's values at positions before its first token: the old conv state, or
+// zeros (prefix[k] is position k - (W-1)); zero before those.
+template <int W>
+__device__ __forceinline__ uint16_t before_row(const uint16_t (&prefix)[W - 1], int t) {
+    uint16_t v = 0;
+#pragma unroll
+    for (int k = 0; k < W - 1; ++k)
+        if (t == k - (W - 1)) v = prefix[k];
+    return v;
+}
+
+// The 8 values of tokens t0 .. t0 + 7 of a row of len tokens, as 4 dwords:
+// one 16-byte load when they all exist and `vec` says the address is aligned,
+// else one by one, past the row zero and (SHIFT: t0 may be negative) positions
+// before it from its prefix.
+template <int W, bool SHIFT>
+__device__ __forceinline__ void load_chunk(const uint16_t *xr, long long t0, long long len, bool vec,
+                                           const uint16_t (&prefix)[W - 1], uint32_t (&dw)[4]) {
+    if (vec && (!SHIFT || t0 >= 0) && t0 + 8 <= len) {
+        const uint4 q = ld_stream(reinterpret_cast<const uint4 *>(xr + t0));
+        dw[0] = q.x; dw[1] = q.y; dw[2] = q.z; dw[3] = q.w;
+        return;
+    }
+    uint16_t e[8];
+#pragma unroll
+    for (int j = 0; j < 8; ++j) e[j] = ((!SHIFT || t0 + j >= 0) && t0 + j < len) ? xr[t0 + j] : 0;
+    if (SHIFT && t0 < 0) {
+#pragma unroll
+        for (int j = 0; j < 8; ++j)
+            if (t0 + j < 0) e[j] = before_row<W>(prefix, static_cast<int>(t0) + j);
+    }
+#pragma unroll
+    for (int j = 0; j < 4; ++j) dw[j] = e[2 * j] | (static_cast<uint32_t>(e[2 * j + 1]) << 16);
+}
+
+// The outputs of that chunk, stored as it was loaded.
+template <bool SHIFT>
+__device__ __forceinline__ void store_chunk(uint16_t *outr, long long t0, long long len, bool vec,
+                                            const float (&o)[8]) {
+    if (vec && (!SHIFT || t0 >= 0) && t0 + 8 <= len) {
+        uint4 q;
+        q.x = pack_h2(o[0], o[1]);
+        q.y = pack_h2(o[2], o[3]);
+        q.z = pack_h2(o[4], o[5]);
+        q.w = pack_h2(o[6], o[7]);
+        st_stream(reinterpret_cast<uint4 *>(outr + t0), q);
+        return;
+    }
+#pragma unroll
+    for (int j = 0; j < 8; ++j)
+        if ((!SHIFT || t0 + j >= 0) && t0 + j < len) outr[t0 + j] = f2h(o[j]);
+}
+
+// Elements between the 16-byte boundary at or before p and p.
+__device__ __forceinline__ int misalign(const uint16_t *p) {
+    return static_cast<int>((reinterpret_cast<uintptr_t>(p) >> 1) & 7);
+}
+
+// Elements between the 128-byte line that holds p and p.
+__device__ __forceinline__ int line_misalign(const uint16_t *p) {
+    return static_cast<int>((reinterpret_cast<uintptr_t>(p) >> 1) & 63);
+}
+
 // Token-contiguous rows ([batch, dim, seqlen] and the reference's
 // [dim, tokens]): one wave streams whole (sequence, channel) rows.  The row is
-// cut into segments of 512 tokens, lane l owning tokens [8l, 8l + 8) of a
+// cut into segments of 512 tokens, lane l owning 8 consecutive tokens of a
 // segment as one 16-byte vector; the loads of up to kSegs segments are issued
 // together, so every lane keeps kSegs vectors in flight.  The W-1 inputs
 // before a lane's tokens are the last values of lane l-1's vector (a lane
 // shuffle), of lane 63 of the previous segment (a readlane) for lane 0, and
 // the carried last values of the previous group of segments, or the prefix
-// (old conv state or zeros), at the start of a row.  A workgroup of 4 waves
-// takes 4 * kRowsPerWave consecutive rows.  Token stride is 1 (x and out).
-// One row per wave: at [8, 4096, 2048] that is 32768 short-lived waves, which
-// keep reads and writes of different waves overlapped (47.5 us); 4 rows per
-// wave made the resident waves load, compute and store in lockstep (58.3 us).
+// (old conv state or zeros), at the start of a row.  Token stride is 1 (x and
+// out).
+//
+// SHIFT (rows that may start off a 16-byte boundary): the cut starts at the
+// boundary at or before the row's first token (m elements before it), so that
+// whole vectors are aligned wherever the row starts, as long as x and out are
+// off by the same amount (they are for equal strides); only the first and last
+// vectors of a row go element by element.  [8, 4096, 2051] 149.6 -> 58.4 us;
+// at [8, 4096, 1000], whose rows are aligned, it would take 35.0 against 30.3.
+//
+// Grid (channels / 4, sequences), 4 waves of one row each: at [8, 4096, 2048]
+// that is 32768 short-lived waves, which keep reads and writes of different
+// waves overlapped (47.5 us); 4 rows per wave made the resident waves load,
+// compute and store in lockstep (58.3 us).
 constexpr int kSegs = 4;
-constexpr int kRowsPerWave = 1;
 
-template <int W, bool SILU>
+template <int W, bool SILU, bool SHIFT>
 __global__ void __launch_bounds__(256) conv1d_rows_kernel(ConvArgs a) {
     constexpr int CH = 8, SEG = 64 * CH;
     const int lane = threadIdx.x & 63;
     const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
-    const long long nrows = static_cast<long long>(a.batch) * a.dim;
-    const long long r0 = (static_cast<long long>(blockIdx.x) * 4 + wave) * kRowsPerWave;
-    for (int rr = 0; rr < kRowsPerWave; ++rr) {
-        const long long r = r0 + rr;
-        if (r >= nrows) return;
-        const int b = static_cast<int>(r / a.dim), d = static_cast<int>(r % a.dim);
-        long long len, xoff, ooff;
-        if (a.qsl != nullptr) {
-            const long long s0 = a.qsl[b];
-            len = a.qsl[b + 1] - s0;
-            xoff = s0 * a.xs;
-            ooff = s0 * a.os;
-        } else {
-            len = a.seq_len;
-            xoff = b * a.xb;
-            ooff = b * a.ob;
-        }
-        const int cidx = a.cidx ? a.cidx[b] : b;
-        if (cidx == a.pad_slot_id || len <= 0) continue;
-        const uint16_t *xr = a.x + xoff + d * a.xd;
-        uint16_t *outr = a.out + ooff + d * a.od;
-        const bool use_state =
-            a.state != nullptr && (a.api_mode == 1 || (a.hinit != nullptr && a.hinit[b] != 0));
-        uint16_t *st = a.state ? a.state + static_cast<long long>(cidx) * a.state_stride + d : nullptr;
-        const bool vec_row = tecoops::aligned(xr, 16) && tecoops::aligned(outr, 16);
-        float wv[W];
+    const int b = blockIdx.y, d = blockIdx.x * 4 + wave;
+    if (d >= a.dim) return;
+    long long len, xoff, ooff;
+    if (a.qsl != nullptr) {
+        const long long s0 = a.qsl[b];
+        len = a.qsl[b + 1] - s0;
+        xoff = s0 * a.xs;
+        ooff = s0 * a.os;
+    } else {
+        len = a.seq_len;
+        xoff = b * a.xb;
+        ooff = b * a.ob;
+    }
+    const int cidx = a.cidx ? a.cidx[b] : b;
+    if (cidx == a.pad_slot_id || len <= 0) return;
+    const uint16_t *xr = a.x + xoff + d * a.xd;
+    uint16_t *outr = a.out + ooff + d * a.od;
+    const bool use_state =
+        a.state != nullptr && (a.api_mode == 1 || (a.hinit != nullptr && a.hinit[b] != 0));
+    uint16_t *st = a.state ? a.state + static_cast<long long>(cidx) * a.state_stride + d : nullptr;
+    const bool vec = !SHIFT || misalign(xr) == misalign(outr);
+    const int m = SHIFT && vec ? misalign(xr) : 0;
+    float wv[W];
 #pragma unroll
-        for (int k = 0; k < W; ++k)
-            wv[k] = h2f(a.w[static_cast<long long>(d) * a.wd + k * a.ww]);
-        const float bv = a.bias ? h2f(a.bias[d]) : 0.0f;
-        // prefix[k]: full_x at position k - (W-1), the old state or zeros
-        uint16_t prefix[W - 1];
+    for (int k = 0; k < W; ++k)
+        wv[k] = h2f(a.w[static_cast<long long>(d) * a.wd + k * a.ww]);
+    const float bv = a.bias ? h2f(a.bias[d]) : 0.0f;
+    // prefix[k]: full_x at position k - (W-1), the old state or zeros
+    uint16_t prefix[W - 1];
 #pragma unroll
-        for (int k = 0; k < W - 1; ++k) prefix[k] = use_state ? st[static_cast<long long>(k) * a.dim] : 0;
-        // carry[k]: full_x at position g0 - 3 + k for the current group start g0
-        float carry[3] = {0.0f, 0.0f, 0.0f};
+    for (int k = 0; k < W - 1; ++k) prefix[k] = use_state ? st[static_cast<long long>(k) * a.dim] : 0;
+    // carry[k]: full_x at position g0 - 3 + k for the current group start g0
+    float carry[3];
 #pragma unroll
-        for (int k = 0; k < W - 1; ++k) carry[3 - (W - 1) + k] = h2f(prefix[k]);
+    for (int k = 0; k < 3; ++k) carry[k] = h2f(before_row<W>(prefix, k - 3 - m));
 
-        for (long long g0 = 0; g0 < len; g0 += kSegs * SEG) {
-            const int nseg = static_cast<int>(min<long long>(kSegs, (len - g0 + SEG - 1) / SEG));
-            uint32_t dw[kSegs][4];
+    for (long long g0 = -m; g0 < len; g0 += kSegs * SEG) {
+        const int nseg = static_cast<int>(min<long long>(kSegs, (len - g0 + SEG - 1) / SEG));
+        uint32_t dw[kSegs][4];
 #pragma unroll
-            for (int u = 0; u < kSegs; ++u) {
-                if (u >= nseg) break;
-                const long long t0 = g0 + u * SEG + lane * CH;
-                if (vec_row && t0 + CH <= len) {
-                    const uint4 q = ld_stream(reinterpret_cast<const uint4 *>(xr + t0));
-                    dw[u][0] = q.x; dw[u][1] = q.y; dw[u][2] = q.z; dw[u][3] = q.w;
-                } else {
-                    uint16_t e[CH];
-#pragma unroll
-                    for (int j = 0; j < CH; ++j) e[j] = (t0 + j < len) ? xr[t0 + j] : 0;
-#pragma unroll
-                    for (int j = 0; j < 4; ++j)
-                        dw[u][j] = e[2 * j] | (static_cast<uint32_t>(e[2 * j + 1]) << 16);
-                }
-            }
-#pragma unroll
-            for (int u = 0; u < kSegs; ++u) {
-                if (u >= nseg) break;
-                const long long t0 = g0 + u * SEG + lane * CH;
-                // tokens t0-3 .. t0-1: lane-1's last three, or for lane 0 the
-                // previous segment's lane 63 (the carry for the first segment)
-                const uint32_t p2 = __shfl_up(dw[u][2], 1, 64);
-                const uint32_t p3 = __shfl_up(dw[u][3], 1, 64);
-                float prev[3] = {hi<f16>(p2), lo<f16>(p3), hi<f16>(p3)};
-                if (lane == 0) {
-                    if (u == 0) {
-                        prev[0] = carry[0]; prev[1] = carry[1]; prev[2] = carry[2];
-                    } else {
-                        const uint32_t q2 = __builtin_amdgcn_readlane(dw[u - 1][2], 63);
-                        const uint32_t q3 = __builtin_amdgcn_readlane(dw[u - 1][3], 63);
-                        prev[0] = hi<f16>(q2); prev[1] = lo<f16>(q3); prev[2] = hi<f16>(q3);
-                    }
-                }
-                float win[W - 1 + CH];
-#pragma unroll
-                for (int k = 0; k < W - 1; ++k) win[k] = prev[3 - (W - 1) + k];
-#pragma unroll
-                for (int j = 0; j < 4; ++j) {
-                    win[W - 1 + 2 * j] = lo<f16>(dw[u][j]);
-                    win[W - 1 + 2 * j + 1] = hi<f16>(dw[u][j]);
-                }
-                float o[CH];
-#pragma unroll
-                for (int j = 0; j < CH; ++j) {
-                    float acc = 0.0f;
-#pragma unroll
-                    for (int k = 0; k < W; ++k) acc += win[j + k] * wv[k];
-                    o[j] = act<SILU>(acc + bv);
-                }
-                if (vec_row && t0 + CH <= len) {
-                    uint4 q;
-                    q.x = pack_h2(o[0], o[1]);
-                    q.y = pack_h2(o[2], o[3]);
-                    q.z = pack_h2(o[4], o[5]);
-                    q.w = pack_h2(o[6], o[7]);
-                    st_stream(reinterpret_cast<uint4 *>(outr + t0), q);
-                } else {
-#pragma unroll
-                    for (int j = 0; j < CH; ++j)
-                        if (t0 + j < len) outr[t0 + j] = f2h(o[j]);
-                }
-            }
-            // the next group starts at g0 + kSegs * SEG only when this group was
-            // full, and then its last three tokens are lane 63's of segment kSegs-1
-            const uint32_t c2 = __builtin_amdgcn_readlane(dw[kSegs - 1][2], 63);
-            const uint32_t c3 = __builtin_amdgcn_readlane(dw[kSegs - 1][3], 63);
-            carry[0] = hi<f16>(c2); carry[1] = lo<f16>(c3); carry[2] = hi<f16>(c3);
+        for (int u = 0; u < kSegs; ++u) {
+            if (u >= nseg) break;
+            load_chunk<W, SHIFT>(xr, g0 + u * SEG + lane * CH, len, vec, prefix, dw[u]);
         }
-        if (lane == 0 && st != nullptr) {
-            uint16_t ns[W - 1];
 #pragma unroll
-            for (int k = 0; k < W - 1; ++k) {
-                const long long src = len - (W - 1) + k;
-                uint16_t old = 0;  // prefix[W - 1 + src] without a dynamic index
+        for (int u = 0; u < kSegs; ++u) {
+            if (u >= nseg) break;
+            // tokens t0-3 .. t0-1: lane-1's last three, or for lane 0 the
+            // previous segment's lane 63 (the carry for the first segment)
+            const uint32_t p2 = __shfl_up(dw[u][2], 1, 64);
+            const uint32_t p3 = __shfl_up(dw[u][3], 1, 64);
+            float prev[3] = {hi<f16>(p2), lo<f16>(p3), hi<f16>(p3)};
+            if (lane == 0) {
+                if (u == 0) {
+                    prev[0] = carry[0]; prev[1] = carry[1]; prev[2] = carry[2];
+                } else {
+                    const uint32_t q2 = __builtin_amdgcn_readlane(dw[u - 1][2], 63);
+                    const uint32_t q3 = __builtin_amdgcn_readlane(dw[u - 1][3], 63);
+                    prev[0] = hi<f16>(q2); prev[1] = lo<f16>(q3); prev[2] = hi<f16>(q3);
+                }
+            }
+            float win[W - 1 + CH];
 #pragma unroll
-                for (int m = 0; m < W - 1; ++m)
-                    if (m == W - 1 + src) old = prefix[m];
-                ns[k] = src >= 0 ? xr[src] : old;
+            for (int k = 0; k < W - 1; ++k) win[k] = prev[3 - (W - 1) + k];
+#pragma unroll
+            for (int j = 0; j < 4; ++j) {
+                win[W - 1 + 2 * j] = lo<f16>(dw[u][j]);
+                win[W - 1 + 2 * j + 1] = hi<f16>(dw[u][j]);
+            }
+            float o[CH];
+#pragma unroll
+            for (int j = 0; j < CH; ++j) {
+                float acc = 0.0f;
+#pragma unroll
+                for (int k = 0; k < W; ++k) acc += win[j + k] * wv[k];
+                o[j] = act<SILU>(acc + bv);
+            }
+            store_chunk<SHIFT>(outr, g0 + u * SEG + lane * CH, len, vec, o);
+        }
+        // the next group starts at g0 + kSegs * SEG only when this group was
+        // full, and then its last three tokens are lane 63's of segment kSegs-1
+        const uint32_t c2 = __builtin_amdgcn_readlane(dw[kSegs - 1][2], 63);
+        const uint32_t c3 = __builtin_amdgcn_readlane(dw[kSegs - 1][3], 63);
+        carry[0] = hi<f16>(c2); carry[1] = lo<f16>(c3); carry[2] = hi<f16>(c3);
+    }
+    if (lane == 0 && st != nullptr) {
+        uint16_t ns[W - 1];
+#pragma unroll
+        for (int k = 0; k < W - 1; ++k) {
+            const long long src = len - (W - 1) + k;
+            ns[k] = src >= 0 ? xr[src] : before_row<W>(prefix, static_cast<int>(src));
+        }
+#pragma unroll
+        for (int k = 0; k < W - 1; ++k) st[static_cast<long long>(k) * a.dim] = ns[k];
+    }
+}
+
+// ------------------------------------- ragged sequences along one token axis
+
+// Index of the sequence that holds token t, or the first one when t lies
+// before it (t and the result wave-uniform; qsl read with scalar loads).
+__device__ __forceinline__ int uniform_seq_of(const int *qsl, int batch, int t) {
+    const auto *q4 = (const __attribute__((address_space(4))) int *)(qsl);
+    int lo = 0, hi = batch - 1;
+    while (lo < hi) {
+        const int mid = (lo + hi + 1) >> 1;
+        if (q4[mid] <= t) lo = mid; else hi = mid - 1;
+    }
+    return lo;
+}
+
+// Token-contiguous rows of a varlen batch ([dim, tokens] with
+// query_start_loc): a channel's sequences lie one after the other, so its row
+// is convolved as one run of tokens, and the first W-1 outputs of each
+// sequence are then redone with the sequence's own past, one sequence per
+// lane.  Cutting the row at every sequence start instead (one wave per
+// sequence and channel) leaves lanes idle in short sequences and pays a
+// wave's set-up, two part vectors and a state update for each: those rows are
+// bound by instructions, not by memory.  16 sequences of 64-2048 tokens (8064
+// in all), dim 4096, 132 MB, µs: one wave per sequence and channel 85.5 with
+// 2-byte accesses off the 16-byte boundary, 65.4 with aligned vectors; one
+// workgroup per channel 36.7.
+//
+// Workgroup: one channel (consecutive channels on one XCD: they share cache
+// lines of the state and the weights); its waves take groups of 4 segments of
+// 512 tokens in turn.  Groups are cut at 128-byte lines of out (m elements
+// before token 0), so that no line is stored in two parts, by 16-byte vectors
+// where x is off the 16-byte boundary by the same amount.  A group's vectors
+// are stored before its sequences' first tokens; new states are written after
+// a barrier, when every old one has been read.
+template <int W, bool SILU>
+__global__ void __launch_bounds__(256) conv1d_axis_kernel(ConvArgs a, int per_xcd) {
+    constexpr int CH = 8, SEG = 64 * CH, GROUP = kSegs * SEG;
+    const int lane = threadIdx.x & 63;
+    const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+    const int d = (blockIdx.x % 8) * per_xcd + blockIdx.x / 8;
+    if (d >= a.dim) return;
+    const auto *q4 = (const __attribute__((address_space(4))) int *)(a.qsl);
+    const int first = q4[0], end = q4[a.batch];  // tokens of the batch
+    const uint16_t *xr = a.x + d * a.xd;
+    uint16_t *outr = a.out + d * a.od;
+    uint16_t *st = a.state ? a.state + d : nullptr;
+    const bool vec = misalign(xr) == misalign(outr);
+    const int m = vec ? line_misalign(outr) : 0;
+    float wv[W];
+#pragma unroll
+    for (int k = 0; k < W; ++k)
+        wv[k] = h2f(a.w[static_cast<long long>(d) * a.wd + k * a.ww]);
+    const float bv = a.bias ? h2f(a.bias[d]) : 0.0f;
+    const auto entry = [&](int b) { return a.cidx ? a.cidx[b] : b; };
+    const auto from_state = [&](int b) {
+        return st != nullptr && (a.api_mode == 1 || (a.hinit != nullptr && a.hinit[b] != 0));
+    };
+    bool skips = false;  // some sequence is skipped
+    if (a.cidx != nullptr) {
+        for (int b = lane; b < a.batch; b += 64) skips |= a.cidx[b] == a.pad_slot_id;
+    } else {
+        skips = a.pad_slot_id >= 0 && a.pad_slot_id < a.batch;
+    }
+    skips = __any(skips);
+
+    for (int g0 = wave * GROUP - m; g0 < end; g0 += GROUP * static_cast<int>(blockDim.x >> 6)) {
+        const int g1 = g0 + GROUP;
+        if (g1 <= first) continue;
+        uint32_t dw[kSegs][4];
+        constexpr uint16_t none[W - 1] = {};
+#pragma unroll
+        for (int u = 0; u < kSegs; ++u) load_chunk<W, true>(xr, g0 + u * SEG + lane * CH, end, vec, none, dw[u]);
+        // tokens g0 - 3 .. g0 - 1, as the upper words of the vector before
+        uint32_t c2 = 0, c3 = 0;
+        if (g0 >= 3) {
+            c2 = static_cast<uint32_t>(xr[g0 - 3]) << 16;
+            c3 = xr[g0 - 2] | (static_cast<uint32_t>(xr[g0 - 1]) << 16);
+        } else if (g0 > 0) {
+            c3 = (g0 > 1 ? xr[g0 - 2] : 0) | (static_cast<uint32_t>(xr[g0 - 1]) << 16);
+        }
+        // the first sequence that can matter here: one that starts within
+        // W - 2 tokens before the group, or holds its first token
+        const int b0 = uniform_seq_of(a.qsl, a.batch, g0 - (W - 2));
+#pragma unroll
+        for (int u = 0; u < kSegs; ++u) {
+            const int t0 = g0 + u * SEG + lane * CH;
+            // tokens t0-3 .. t0-1: lane-1's last three (wave_shr:1), lane 0
+            // those of the previous segment's lane 63 or before the group
+            if (u > 0) {
+                c2 = __builtin_amdgcn_readlane(dw[u - 1][2], 63);
+                c3 = __builtin_amdgcn_readlane(dw[u - 1][3], 63);
+            }
+            const uint32_t p2 = __builtin_amdgcn_update_dpp(c2, dw[u][2], 0x138, 0xF, 0xF, false);
+            const uint32_t p3 = __builtin_amdgcn_update_dpp(c3, dw[u][3], 0x138, 0xF, 0xF, false);
+            const float prev[3] = {hi<f16>(p2), lo<f16>(p3), hi<f16>(p3)};
+            float win[W - 1 + CH];  // win[e]: token t0 - (W-1) + e
+#pragma unroll
+            for (int k = 0; k < W - 1; ++k) win[k] = prev[3 - (W - 1) + k];
+#pragma unroll
+            for (int j = 0; j < 4; ++j) {
+                win[W - 1 + 2 * j] = lo<f16>(dw[u][j]);
+                win[W - 1 + 2 * j + 1] = hi<f16>(dw[u][j]);
+            }
+            float o[CH];
+#pragma unroll
+            for (int j = 0; j < CH; ++j) {
+                float acc = 0.0f;
+#pragma unroll
+                for (int k = 0; k < W; ++k) acc += win[j + k] * wv[k];
+                o[j] = act<SILU>(acc + bv);
+            }
+            uint32_t ok = 0xff;  // tokens of this lane that are stored
+            if (skips) {
+                for (int b = b0; b < a.batch && q4[b] < t0 - lane * CH + SEG; ++b) {
+                    if (entry(b) != a.pad_slot_id) continue;
+                    const int lo8 = min(max(q4[b] - t0, 0), CH), hi8 = min(max(q4[b + 1] - t0, 0), CH);
+                    ok &= ~(((1u << hi8) - 1u) & ~((1u << lo8) - 1u));
+                }
+            }
+            if (ok == 0xff && t0 >= first) {
+                store_chunk<true>(outr, t0, end, vec, o);
+            } else if (ok != 0) {
+#pragma unroll
+                for (int j = 0; j < CH; ++j)
+                    if ((ok >> j & 1) && t0 + j >= first && t0 + j < end) outr[t0 + j] = f2h(o[j]);
+            }
+        }
+        // The tokens of this group that are among the first W-1 of their
+        // sequence, over the values just stored (which have to be there
+        // first: another lane stored them).
+        __builtin_amdgcn_fence(__ATOMIC_RELEASE, "workgroup");
+        for (int base = b0; base < a.batch && q4[base] < g1; base += 64) {
+            const int b = base + lane;
+            if (b >= a.batch) continue;
+            const int s = a.qsl[b], e = a.qsl[b + 1], c = entry(b);
+            if (s >= g1 || s < g0 - (W - 2) || e <= s || c == a.pad_slot_id) continue;
+            // v[i]: full_x at position i - (W-1) of the sequence
+            float v[2 * (W - 1)];
+#pragma unroll
+            for (int k = 0; k < W - 1; ++k) v[k] = 0.0f;
+            if (from_state(b)) {
+#pragma unroll
+                for (int k = 0; k < W - 1; ++k)
+                    v[k] = h2f(st[static_cast<long long>(c) * a.state_stride +
+                                  static_cast<long long>(k) * a.dim]);
             }
 #pragma unroll
-            for (int k = 0; k < W - 1; ++k) st[static_cast<long long>(k) * a.dim] = ns[k];
+            for (int j = 0; j < W - 1; ++j) v[W - 1 + j] = s + j < e ? h2f(xr[s + j]) : 0.0f;
+#pragma unroll
+            for (int j = 0; j < W - 1; ++j) {
+                float acc = 0.0f;
+#pragma unroll
+                for (int k = 0; k < W; ++k) acc += v[j + k] * wv[k];
+                if (s + j >= g0 && s + j < min(g1, e)) outr[s + j] = f2h(act<SILU>(acc + bv));
+            }
         }
+    }
+    if (st == nullptr) return;
+    __syncthreads();
+    for (int b = threadIdx.x; b < a.batch; b += blockDim.x) {
+        const int s = a.qsl[b], e = a.qsl[b + 1], c = entry(b);
+        if (c == a.pad_slot_id || e <= s) continue;
+        uint16_t *sb = st + static_cast<long long>(c) * a.state_stride;
+        uint16_t ns[W - 1];
+#pragma unroll
+        for (int k = 0; k < W - 1; ++k) {
+            const int src = e - (W - 1) + k;
+            ns[k] = src >= s ? xr[src]
+                    : from_state(b) ? sb[static_cast<long long>(src - s + W - 1) * a.dim] : 0;
+        }
+#pragma unroll
+        for (int k = 0; k < W - 1; ++k) sb[static_cast<long long>(k) * a.dim] = ns[k];
     }
 }
 
@@ -782,6 +998,22 @@ bool tokens_layout(const ConvArgs &a) {
 // 18.3 / 15.7 us.  One token: 8 us against 134 us with one row per wave.
 constexpr long long kShortLenNear = 12, kShortLenFar = 4;
 
+// Every row of x and out starts on a 16-byte boundary.
+bool rows_aligned(const ConvArgs &a) {
+    return a.qsl == nullptr && tecoops::aligned(a.x, 16) && tecoops::aligned(a.out, 16) &&
+           a.xd % 8 == 0 && a.xb % 8 == 0 && a.od % 8 == 0 && a.ob % 8 == 0;
+}
+
+// Elements (tokens x channels) from which a varlen batch of token-contiguous
+// rows runs along the whole token axis (conv1d_axis_kernel), sequences short
+// enough for conv1d_short_kernel aside.  µs grouped or per-sequence rows /
+// token axis: dim 4096, 4 x 35 tokens 8.2 / 10.7, 8 x 16 8.6 / 11.0, 64 x 4.5
+// 16.1 / 14.6, 8 x 85 14.4 / 13.4, 4 x 248 16.3 / 12.0, 64 x 10 22.1 / 15.7,
+// 64 x 40 43.5 / 27.1, 32 x 170 74.9 / 31.9, 32 x 274 112.5 / 53.1, 8 x 1950
+// 139.7 / 57.5; dim 1024, 64 x 10 8.1 / 8.7, 64 x 20 9.1 / 9.0, 64 x 39 13.6 /
+// 10.4.
+constexpr long long kAxisMinElems = 1 << 20;
+
 template <int W, bool SILU>
 void launch(const ConvArgs &a0, bool seq_contig, long long max_len, hipStream_t s) {
     ConvArgs a = a0;
@@ -806,6 +1038,16 @@ void launch(const ConvArgs &a0, bool seq_contig, long long max_len, hipStream_t 
         hipLaunchKernelGGL((conv1d_short_kernel<W, SILU>), dim3(grid), dim3(256), 0, s, a);
         return;
     }
+    // (its waves read tokens that others' outputs would overwrite in place)
+    if (seq_contig && a.qsl != nullptr && a.x != a.out && max_len * a.dim >= kAxisMinElems) {
+        // groups of tokens of a channel, four at a time
+        const long long groups = (max_len + 7 + kSegs * 512 - 1) / (kSegs * 512);
+        const unsigned per_xcd = tecoops::ceil_div(a.dim, 8);
+        hipLaunchKernelGGL((conv1d_axis_kernel<W, SILU>), dim3(8 * per_xcd),
+                           dim3(64 * static_cast<unsigned>(groups < 4 ? groups : 4)), 0, s, a,
+                           static_cast<int>(per_xcd));
+        return;
+    }
     if (seq_contig && mean_len <= 256) {
         // short rows: 16, 8, 4 or 2 rows per wave (segments of 32, 64, 128
         // and 256 tokens)
@@ -823,10 +1065,11 @@ void launch(const ConvArgs &a0, bool seq_contig, long long max_len, hipStream_t 
         return;
     }
     if (seq_contig) {
-        (void)max_len;
-        const long long rows = static_cast<long long>(a.batch) * a.dim;
-        const unsigned grid = static_cast<unsigned>(tecoops::ceil_div(rows, 4LL * kRowsPerWave));
-        hipLaunchKernelGGL((conv1d_rows_kernel<W, SILU>), dim3(grid), dim3(256), 0, s, a);
+        const dim3 grid(tecoops::ceil_div(a.dim, 4), a.batch);
+        if (rows_aligned(a))
+            hipLaunchKernelGGL((conv1d_rows_kernel<W, SILU, false>), grid, dim3(256), 0, s, a);
+        else
+            hipLaunchKernelGGL((conv1d_rows_kernel<W, SILU, true>), grid, dim3(256), 0, s, a);
     } else {
         constexpr int CH = 16;
         a.nchunks = static_cast<int>((max_len + CH - 1) / CH);
