@@ -225,7 +225,11 @@ tecoopsStatus_t tecoopsReshapeAndCacheEx(tecoopsHandle_t handle,
  * or call tecoopsFlashAttentionNoAlloc there.  A workspace must hold
  * tecoopsGetFlashAttentionWorkspaceSize() bytes for the same batch, heads,
  * head size, max_seqlen_q and max_seqlen_k, and max_seqlen_k must then be > 0
- * (it sizes the split-KV partials). */
+ * (it sizes the split-KV partials).  A prefill without a workspace whose
+ * longest context outweighs the rest (chunks of prompts over cached context)
+ * splits its keys too, in up to 128 MiB of the handle's scratch per stream;
+ * under capture, on more streams than the handle keeps scratch for, or where no
+ * memory is free it runs unsplit, to the same results up to rounding. */
 tecoopsStatus_t tecoopsFlashAttentionEx(tecoopsHandle_t handle,
                                         int max_seqlen_q, int max_seqlen_k,
                                         const int *q_seq_lens, const int *cu_seqlens_q,
@@ -245,8 +249,8 @@ tecoopsStatus_t tecoopsFlashAttentionEx(tecoopsHandle_t handle,
 /* Flash attention that allocates nothing, for callers that cannot allocate
  * device memory (code under HIP graph capture, tight serving loops, harnesses
  * that forbid hipMalloc).  No counterpart in the reference.  Arguments and
- * results are those of tecoopsFlashAttentionEx without a workspace: the
- * split-KV partials of decode go to a static device array of 64 MiB per GPU
+ * results are those of tecoopsFlashAttentionEx without a workspace (a prefill
+ * that it splits runs unsplit here, which rounds differently): the split-KV partials of decode go to a static device array of 64 MiB per GPU
  * (held until the process ends) instead of the handle's scratch, and a call
  * whose decode plan needs more returns TECOOPS_STATUS_BAD_PARAM.  Every call
  * on a GPU shares that array: calls that overlap on one GPU (different

@@ -41,6 +41,7 @@ SOURCES = [
     "gemv.hip",
     "gemv_batch.hip",
     "flash_attention.hip",
+    "fa_split.hip",
     "fa_noalloc.hip",
 ]
 
@@ -58,6 +59,7 @@ CFLAGS = [
 # scores are -inf), so the softmax max tree needs no NaN canonicalisation.
 EXTRA_FLAGS = {
     "flash_attention.hip": ["-fno-honor-nans"],
+    "fa_split.hip": ["-fno-honor-nans"],
 }
 
 
@@ -70,7 +72,8 @@ EXTRA_FLAGS = {
 # flash_attention.hip and gemv_batch.hip wait for their copies by counting only
 # younger copies (inline assembly, which the compiler keeps in order), so only
 # their use of M0 is checked.
-COPY_WAIT_CHECKED = {"gemv.hip": True, "gemv_batch.hip": False, "flash_attention.hip": False}
+COPY_WAIT_CHECKED = {"gemv.hip": True, "gemv_batch.hip": False, "flash_attention.hip": False,
+                     "fa_split.hip": False}
 
 
 def check_copy_waits(asm_text, src="", waits=True):

@@ -125,4 +125,9 @@ inline int device_cus() {
 // handle's current stream, for an op about to be enqueued there.
 tecoopsStatus_t handle_scratch(tecoopsHandle_t handle, size_t bytes, void **out);
 
+// The same for an op that can do without: nullptr while the stream is
+// captured, when no memory is free, and when another stream would have to
+// give up its buffer.
+void *handle_scratch_if_any(tecoopsHandle_t handle, size_t bytes);
+
 }  // namespace tecoops

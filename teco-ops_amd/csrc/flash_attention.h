@@ -33,6 +33,7 @@ struct FaParams {
     float *ws_o;         // [B][Hkv][max_splits][ncols][D]
     float *ws_ml;        // [B][Hkv][max_splits][ncols][2]
     int split_len, max_splits, rq, ncols;
+    void *ws_plan;       // split prefill: the plan (the states are in ws_o)
 };
 
 // Launch shape.  rq is the host's bound on q_len (routing and grid height),
@@ -44,10 +45,20 @@ struct Plan {
     int rq, rk, ncols, split_len, max_splits;
 };
 
+// Prefill over split keys (fa_split.hip): `slots` pieces share the batch's
+// work, none shorter than `least` keys; wide selects the 12-wave kernels.
+// slots 0: not split.
+struct SplitArgs {
+    int slots, least, wide;
+};
+constexpr int kSplitMaxBatch = 64;        // sequences of a split prefill
+constexpr size_t kSplitPlanBytes = 2048;  // the workspace starts with the plan
+
 // A validated call: kernel parameters, launch shape and element type.
 struct FaCall {
     FaParams p;
     Plan pl;
+    SplitArgs split;  // the split prefill the call may take, given a workspace
     int D;
     bool bf16;
 };
@@ -65,6 +76,11 @@ tecoopsStatus_t prepare(tecoopsHandle_t handle, int max_seqlen_q, int max_seqlen
 
 // Bytes of split-KV partials the call needs (0 for prefill).
 size_t workspace_bytes(const FaCall &c);
+
+// Bytes of partial states of a split prefill, and its launch (p.ws_o holds
+// them).
+size_t split_bytes(const SplitArgs &a, int D);
+tecoopsStatus_t launch_split(hipStream_t s, const FaParams &p, const SplitArgs &a, int D, bool bf16);
 
 // Enqueues the call on stream s, its split-KV partials in ws.
 tecoopsStatus_t launch(hipStream_t s, FaCall &c, void *ws);

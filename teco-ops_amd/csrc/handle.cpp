@@ -224,22 +224,21 @@ bool reserve_lds(const void *kernel, size_t bytes) {
     return true;
 }
 
-tecoopsStatus_t handle_scratch(tecoopsHandle_t handle, size_t bytes, void **out) {
-    // A graph captured from this stream would keep the slot's address, and a
-    // later call may free the slot (a larger plan grows it, a ninth stream
-    // takes it over), leaving the graph writing freed memory.  Under capture
-    // the caller passes a workspace or uses the allocation-free entry point.
+namespace {
+
+// Whether work enqueued on the stream is being captured into a graph.
+bool stream_captured(hipStream_t stream) {
     hipStreamCaptureStatus cs = hipStreamCaptureStatusNone;
-    if (hipStreamIsCapturing(handle->stream, &cs) != hipSuccess) {
+    if (hipStreamIsCapturing(stream, &cs) != hipSuccess) {
         (void)hipGetLastError();
-        cs = hipStreamCaptureStatusNone;
+        return false;
     }
-    if (cs != hipStreamCaptureStatusNone) {
-        TECO_ERROR("the handle's split-KV scratch cannot be used while its stream is captured: "
-                   "pass a workspace (tecoopsFlashAttentionEx) or call "
-                   "tecoopsFlashAttentionNoAlloc");
-        return TECOOPS_STATUS_NOT_SUPPORTED;
-    }
+    return cs != hipStreamCaptureStatusNone;
+}
+
+// The buffer of the handle's current stream, of at least `bytes`; take_over:
+// from the least recently used stream if no slot is free.
+tecoopsStatus_t scratch_slot(tecoopsHandle_t handle, size_t bytes, bool take_over, void **out) {
     if (bytes == 0) bytes = 256;
     ScratchSlot *slot = nullptr;
     for (ScratchSlot &sl : handle->scratch)
@@ -253,6 +252,7 @@ tecoopsStatus_t handle_scratch(tecoopsHandle_t handle, size_t bytes, void **out)
             }
             if (sl.last_use < slot->last_use) slot = &sl;
         }
+        if (slot->ptr != nullptr && !take_over) return TECOOPS_STATUS_ALLOC_FAILED;
         // A buffer taken over from another stream may still be read by work
         // enqueued there: free it (hipFree waits for the device) and let the
         // allocation below start afresh.
@@ -288,6 +288,38 @@ tecoopsStatus_t handle_scratch(tecoopsHandle_t handle, size_t bytes, void **out)
     slot->last_use = ++handle->uses;
     *out = slot->ptr;
     return TECOOPS_STATUS_SUCCESS;
+}
+
+}  // namespace
+
+tecoopsStatus_t handle_scratch(tecoopsHandle_t handle, size_t bytes, void **out) {
+    // A graph captured from this stream would keep the slot's address, and a
+    // later call may free the slot (a larger plan grows it, a ninth stream
+    // takes it over), leaving the graph writing freed memory.  Under capture
+    // the caller passes a workspace or uses the allocation-free entry point.
+    if (stream_captured(handle->stream)) {
+        TECO_ERROR("the handle's split-KV scratch cannot be used while its stream is captured: "
+                   "pass a workspace (tecoopsFlashAttentionEx) or call "
+                   "tecoopsFlashAttentionNoAlloc");
+        return TECOOPS_STATUS_NOT_SUPPORTED;
+    }
+    return scratch_slot(handle, bytes, true, out);
+}
+
+void *handle_scratch_if_any(tecoopsHandle_t handle, size_t bytes) {
+    void *out = nullptr;
+    if (stream_captured(handle->stream)) return nullptr;
+    // Another thread may be capturing its stream in the global mode, in which
+    // an allocation here would end that capture; this one is no part of it.
+    hipStreamCaptureMode mode = hipStreamCaptureModeRelaxed;
+    const bool relaxed = hipThreadExchangeStreamCaptureMode(&mode) == hipSuccess;
+    if (!relaxed) {
+        (void)hipGetLastError();
+        return nullptr;
+    }
+    if (scratch_slot(handle, bytes, false, &out) != TECOOPS_STATUS_SUCCESS) out = nullptr;
+    if (hipThreadExchangeStreamCaptureMode(&mode) != hipSuccess) (void)hipGetLastError();
+    return out;
 }
 
 }  // namespace tecoops

@@ -169,7 +169,10 @@ void flash_attn_varlen_func(const Tensor &q, const Tensor &k, const Tensor &v,
         q_hint = static_cast<int>(std::min<int64_t>(std::max(max_seqlen_q, q_mean), 0x7fffffff));
         k_hint = static_cast<int>(max_seqlen_k > 0 ? std::min<int64_t>(max_seqlen_k, cap) : cap);
         size_t bytes = 0;
-        if (k_hint > 0 &&
+        // a workspace is for the decode route (at most 32 query columns per kv
+        // head); a prefill uses the handle's scratch where it splits its keys
+        const bool decode = k.size(1) > 0 && q.size(1) / k.size(1) * static_cast<int64_t>(q_hint) <= 32;
+        if (decode && k_hint > 0 &&
             tecoopsGetFlashAttentionWorkspaceSize(static_cast<int>(batch), static_cast<int>(q.size(1)),
                                                   static_cast<int>(q.size(2)), q_hint, k_hint,
                                                   &bytes) == TECOOPS_STATUS_SUCCESS &&
