@@ -250,11 +250,12 @@ tecoopsStatus_t tecoopsFlashAttentionEx(tecoopsHandle_t handle,
  * device memory (code under HIP graph capture, tight serving loops, harnesses
  * that forbid hipMalloc).  No counterpart in the reference.  Arguments and
  * results are those of tecoopsFlashAttentionEx without a workspace (a prefill
- * that it splits runs unsplit here, which rounds differently): the split-KV partials of decode go to a static device array of 64 MiB per GPU
- * (held until the process ends) instead of the handle's scratch, and a call
- * whose decode plan needs more returns TECOOPS_STATUS_BAD_PARAM.  Every call
- * on a GPU shares that array: calls that overlap on one GPU (different
- * streams, threads or handles) race and must be ordered by the caller. */
+ * that it splits runs unsplit here, which rounds differently): the split-KV
+ * partials of decode go to a static device array of 64 MiB per GPU (held until
+ * the process ends) instead of the handle's scratch, and a call whose decode
+ * plan needs more returns TECOOPS_STATUS_BAD_PARAM.  Every call on a GPU
+ * shares that array: calls that overlap on one GPU (different streams, threads
+ * or handles) race and must be ordered by the caller. */
 tecoopsStatus_t tecoopsFlashAttentionNoAlloc(tecoopsHandle_t handle,
                                              int max_seqlen_q, int max_seqlen_k,
                                              const int *q_seq_lens, const int *cu_seqlens_q,

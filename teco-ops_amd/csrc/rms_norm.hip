@@ -7,13 +7,12 @@
 //         unrounded v; y = T(float(T(v)) * rstd * w)
 // fp32 accumulation throughout.
 //
-// gfx950 design: rows up to 8192 elements (16-byte aligned, D % 8 == 0) run
-// one wave per row: each lane keeps its chunks of the row in registers
-// between the reduction and the output pass, so x (and r) are read from HBM
-// exactly once and the sum of squares is a wave-wide xor-shuffle reduction
-// (no LDS, no barrier).  Rows up to 16384 use a 256-lane workgroup per row
-// with an LDS reduction across its 4 waves.  Other rows (D % 8 != 0,
-// misaligned, wider) take a two-pass element loop (second read hits L2).  HBM-bound:
+// gfx950 design: rows of up to 16384 elements (16-byte aligned, D % 8 == 0) are
+// kept in registers between the reduction and the output pass, so x (and r)
+// are read from HBM exactly once.  Narrow rows and many of up to 4096 run one
+// wave per row (a wave-wide xor-shuffle reduction, no LDS, no barrier), the
+// others a workgroup per row (dispatch()).  Other rows (D % 8 != 0, misaligned,
+// wider) take a two-pass element loop (second read hits L2).  HBM-bound:
 // algorithmic bytes = 2*N*D*2 + 2*D (+ 2*N*D*2 for the add variant).
 #include "common.h"
 #include "device.h"
@@ -23,6 +22,7 @@ namespace {
 using namespace tecoops::dev;
 
 constexpr int kThreads = 256;
+constexpr int kRowThreads = 512;
 
 __device__ __forceinline__ float block_sum(float v, float *red) {
     v = wave_sum(v);
@@ -35,44 +35,44 @@ __device__ __forceinline__ float block_sum(float v, float *red) {
     return s;
 }
 
+// A workgroup per row, VPT 16-byte chunks per lane.  Every load of the row is
+// asked for before the first use, the weight's too: with few rows the time is
+// one trip to memory, the reduction and the stores (8 x 4096 with residual:
+// 2.7 us, and a row of 512 takes 1.8; one wave per row waits for x, r
+// and w in turn over 8 chunks per lane, 8.8).
 template <typename T, int VPT, bool ADD>
-__global__ void __launch_bounds__(kThreads)
-rms_norm_vec(const uint4 *__restrict__ x, const uint4 *__restrict__ w, const uint4 *__restrict__ r,
+__global__ void __launch_bounds__(kRowThreads)
+rms_norm_row(const uint4 *__restrict__ x, const uint4 *__restrict__ w, const uint4 *__restrict__ r,
              uint4 *__restrict__ y, uint4 *__restrict__ r_out, int vec_per_row, int hidden,
              float eps) {
-    __shared__ float red[kThreads / 64];
-    const long long row = blockIdx.x;
-    const uint4 *xr = x + row * vec_per_row;
-    uint4 v[VPT];
-    float ss = 0.0f;
+    __shared__ float red[kRowThreads / 64];
+    const long long row = static_cast<long long>(blockIdx.x) * vec_per_row;
+    uint4 v[VPT], b[VPT], wv[VPT];
 #pragma unroll
     for (int j = 0; j < VPT; ++j) {
         const int c = threadIdx.x + j * blockDim.x;
+        v[j] = b[j] = wv[j] = uint4{0, 0, 0, 0};
         if (c < vec_per_row) {
-            uint4 a = xr[c];
+            v[j] = x[row + c];
+            if (ADD) b[j] = r[row + c];
+            wv[j] = w[c];
+        }
+    }
+    float ss = 0.0f;
+#pragma unroll
+    for (int j = 0; j < VPT; ++j) {
+        uint32_t *pa = reinterpret_cast<uint32_t *>(&v[j]);
+        const uint32_t *pb = reinterpret_cast<const uint32_t *>(&b[j]);
+#pragma unroll
+        for (int q = 0; q < 4; ++q) {
+            float s0 = lo<T>(pa[q]), s1 = hi<T>(pa[q]);
             if (ADD) {
-                const uint4 b = r[row * vec_per_row + c];
-                uint32_t *pa = reinterpret_cast<uint32_t *>(&a);
-                const uint32_t *pb = reinterpret_cast<const uint32_t *>(&b);
-#pragma unroll
-                for (int q = 0; q < 4; ++q) {
-                    const float s0 = lo<T>(pa[q]) + lo<T>(pb[q]);
-                    const float s1 = hi<T>(pa[q]) + hi<T>(pb[q]);
-                    ss += s0 * s0;
-                    ss += s1 * s1;
-                    pa[q] = pack<T>(s0, s1);
-                }
-                r_out[row * vec_per_row + c] = a;
-            } else {
-                const uint32_t *pa = reinterpret_cast<const uint32_t *>(&a);
-#pragma unroll
-                for (int q = 0; q < 4; ++q) {
-                    const float s0 = lo<T>(pa[q]), s1 = hi<T>(pa[q]);
-                    ss += s0 * s0;
-                    ss += s1 * s1;
-                }
+                s0 += lo<T>(pb[q]);
+                s1 += hi<T>(pb[q]);
+                pa[q] = pack<T>(s0, s1);
             }
-            v[j] = a;
+            ss += s0 * s0;
+            ss += s1 * s1;
         }
     }
     const float total = block_sum(ss, red);
@@ -81,16 +81,16 @@ rms_norm_vec(const uint4 *__restrict__ x, const uint4 *__restrict__ w, const uin
     for (int j = 0; j < VPT; ++j) {
         const int c = threadIdx.x + j * blockDim.x;
         if (c < vec_per_row) {
-            const uint4 wv = w[c];
             const uint32_t *pa = reinterpret_cast<const uint32_t *>(&v[j]);
-            const uint32_t *pw = reinterpret_cast<const uint32_t *>(&wv);
+            const uint32_t *pw = reinterpret_cast<const uint32_t *>(&wv[j]);
             uint4 o;
             uint32_t *po = reinterpret_cast<uint32_t *>(&o);
 #pragma unroll
             for (int q = 0; q < 4; ++q)
                 po[q] = pack<T>(lo<T>(pa[q]) * rstd * lo<T>(pw[q]),
                                 hi<T>(pa[q]) * rstd * hi<T>(pw[q]));
-            y[row * vec_per_row + c] = o;
+            if (ADD) r_out[row + c] = v[j];
+            y[row + c] = o;
         }
     }
 }
@@ -198,12 +198,13 @@ void launch_wave(const void *x, const void *w, const void *r, void *y, void *ro,
 }
 
 template <typename T, int VPT, bool ADD>
-void launch_vec(int threads, const void *x, const void *w, const void *r, void *y, void *ro,
-                int rows, int hidden, float eps, hipStream_t s) {
-    hipLaunchKernelGGL((rms_norm_vec<T, VPT, ADD>), dim3(rows), dim3(threads), 0, s,
+void launch_row(const void *x, const void *w, const void *r, void *y, void *ro, int rows, int hidden,
+                float eps, hipStream_t s) {
+    const int nvec = hidden / 8, waves = (nvec + 64 * VPT - 1) / (64 * VPT);
+    hipLaunchKernelGGL((rms_norm_row<T, VPT, ADD>), dim3(rows), dim3(64 * waves), 0, s,
                        static_cast<const uint4 *>(x), static_cast<const uint4 *>(w),
                        static_cast<const uint4 *>(r), static_cast<uint4 *>(y),
-                       static_cast<uint4 *>(ro), hidden / 8, hidden, eps);
+                       static_cast<uint4 *>(ro), nvec, hidden, eps);
 }
 
 template <typename T, bool ADD>
@@ -214,22 +215,23 @@ tecoopsStatus_t dispatch(tecoopsHandle_t handle, const void *x, const void *w, c
     for (const void *p : {x, w, r, static_cast<const void *>(y), static_cast<const void *>(ro)})
         if (p != nullptr) vec = vec && tecoops::aligned(p, 16);
     const int nvec = hidden / 8;
-    if (vec && nvec <= 64 * 16) {
-        // up to 16 chunks (8 KiB of fp16 row at 4096 hidden = 8 chunks) per lane
+    // Measured on bf16 rows, us, wave per row / workgroup per row: 8 rows of
+    // 4096 with residual 8.8 / 2.7, 8 of 1024 2.6 / 2.0, 1024 of 1024 3.4 / 3.1,
+    // 2048 of 1024 3.8 / 3.9, 1024 of 4096 7.3 / 5.6, 4096 of 4096 13.3 / 14.3,
+    // with residual 26.2 / 25.5, 4096 of 8192 29.5 / 22.6.  One chunk per lane
+    // (up to 512 wide) is the same trip to memory either way, and the wave has
+    // no barrier: 8 rows 2.0 / 2.0, 8192 rows 4.7 / 5.4.
+    const bool by_row = nvec > 512 || (nvec > 64 && (rows <= 1024 || (ADD && nvec >= 256)));
+    if (vec && nvec <= 4 * kRowThreads && by_row) {
+        if (nvec <= kRowThreads) launch_row<T, 1, ADD>(x, w, r, y, ro, rows, hidden, eps, s);
+        else if (nvec <= 2 * kRowThreads) launch_row<T, 2, ADD>(x, w, r, y, ro, rows, hidden, eps, s);
+        else launch_row<T, 4, ADD>(x, w, r, y, ro, rows, hidden, eps, s);
+    } else if (vec && nvec <= 64 * 8) {
         const int vpt = (nvec + 63) / 64;
         if (vpt <= 1) launch_wave<T, 1, ADD>(x, w, r, y, ro, rows, hidden, eps, s);
         else if (vpt <= 2) launch_wave<T, 2, ADD>(x, w, r, y, ro, rows, hidden, eps, s);
         else if (vpt <= 4) launch_wave<T, 4, ADD>(x, w, r, y, ro, rows, hidden, eps, s);
-        else if (vpt <= 8) launch_wave<T, 8, ADD>(x, w, r, y, ro, rows, hidden, eps, s);
-        else launch_wave<T, 16, ADD>(x, w, r, y, ro, rows, hidden, eps, s);
-    } else if (vec && nvec <= kThreads * 8) {
-        // Narrow rows use one wave; wide rows 256 lanes with up to 8 chunks each.
-        const int threads = nvec <= 64 ? 64 : (nvec <= 128 ? 128 : kThreads);
-        const int vpt = (nvec + threads - 1) / threads;
-        if (vpt <= 1) launch_vec<T, 1, ADD>(threads, x, w, r, y, ro, rows, hidden, eps, s);
-        else if (vpt <= 2) launch_vec<T, 2, ADD>(threads, x, w, r, y, ro, rows, hidden, eps, s);
-        else if (vpt <= 4) launch_vec<T, 4, ADD>(threads, x, w, r, y, ro, rows, hidden, eps, s);
-        else launch_vec<T, 8, ADD>(threads, x, w, r, y, ro, rows, hidden, eps, s);
+        else if constexpr (!ADD) launch_wave<T, 8, ADD>(x, w, r, y, ro, rows, hidden, eps, s);
     } else {
         hipLaunchKernelGGL((rms_norm_scalar<T, ADD>), dim3(rows), dim3(kThreads), 0, s,
                            static_cast<const uint16_t *>(x), static_cast<const uint16_t *>(w),
