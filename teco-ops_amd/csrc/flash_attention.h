@@ -33,6 +33,7 @@ struct FaParams {
     float *ws_o;         // [B][Hkv][max_splits][ncols][D]
     float *ws_ml;        // [B][Hkv][max_splits][ncols][2]
     int split_len, max_splits, rq, ncols;
+    bool direct;         // decode workgroups take their item in grid order
     void *ws_plan;       // split prefill: the plan (the states are in ws_o)
 };
 

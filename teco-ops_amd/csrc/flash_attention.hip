@@ -390,13 +390,16 @@ __global__ void __launch_bounds__(256, D > 128 ? 1 : 2) fa_decode_kernel(FaParam
     if (blockIdx.x == 0 && blockIdx.y == 0) zero_tail_rows(p, D);
     int b, kvh, split, L, S;
     long long q_off;
-    if (p.batch <= 64) {
+    if (p.batch <= 64 && !p.direct) {
         if (!decode_item(p, blockIdx.y * gridDim.x + blockIdx.x, b, kvh, split, q_off, L, S))
             return;
     } else {
         // Larger batches keep the grid's order, (sequence, kv head) by split:
         // with hundreds of items per CU the tail is short, and a scan over
-        // every sequence in each workgroup would cost more than it saves.
+        // every sequence in each workgroup would cost more than it saves.  So
+        // do grids of no more workgroups than CUs, which all run at once (4
+        // sequences of 255..4095 keys 12.8 / 11.0 us; up to two per CU even
+        // lengths still gain 0.6, 8 uneven ones lose 2.5).
         b = turned_column(blockIdx.x / p.Hkv, blockIdx.y, p.batch);
         kvh = blockIdx.x % p.Hkv;
         split = blockIdx.y;
@@ -446,85 +449,101 @@ __global__ void __launch_bounds__(256, D > 128 ? 1 : 2) fa_decode_kernel(FaParam
     });
 }
 
-// Merges the split partials of (b, kv head) into the output rows.  The
-// splits' (m, l) are staged in LDS once, one thread per column turns them into
-// normalised weights, and each output element then sums its splits' partial
-// O with independent loads.  Split counts beyond the LDS staging capacity
-// take a two-pass loop over global memory instead.
-constexpr int kCombineStage = 2048;  // (split, column) pairs staged in LDS
+// Merges the split partials of (b, kv head) into the output rows: a row of
+// lanes, four dims each, takes every ways-th split of one column, kAhead loads
+// at a time.  The first ones are asked for before the lengths are known (splits
+// a sequence does not have are skipped afterwards), so with up to kAhead *
+// ways splits the kernel is one trip to memory; the ways meet in LDS.  One
+// workgroup per (b, kv head), with the weights staged first and one thread per
+// element, took 4.4 us of 8 sequences of 255..4095 keys and 27 of 1 x 32768 by
+// 1 kv head (8 heads, 64 splits; the call 43 us, now 20).
+constexpr int kAhead = 4;
+
+template <int D>
+constexpr int combine_rows() {  // rows of lanes in a workgroup (a power of two)
+    int n = 1;
+    while (2 * n * (D / 4) <= 256) n *= 2;
+    return n;
+}
 
 template <typename T, int D>
-__global__ void __launch_bounds__(256) fa_decode_combine_kernel(FaParams p) {
-    __shared__ float wgt[kCombineStage];  // [split][column]: m, then weight / total l
-    __shared__ float lsp[kCombineStage];  // [split][column]: l
+__global__ void __launch_bounds__(256) fa_decode_combine_kernel(FaParams p, int ways) {
+    constexpr int ROWS = combine_rows<D>(), V = D / 4;
+    // (a caller's workspace need not be aligned to 16 bytes)
+    typedef float4_t __attribute__((aligned(4))) float4_u;
+    typedef float2_t __attribute__((aligned(4))) float2_u;
+    __shared__ __attribute__((aligned(16))) float4_t acc_of[ROWS * V];
+    __shared__ float m_of[ROWS], l_of[ROWS];
     const int kvh = blockIdx.x % p.Hkv;
     const int b = blockIdx.x / p.Hkv;
+    const int slot = threadIdx.x / V, e = threadIdx.x % V;
+    const int way = slot % ways, c = blockIdx.y * (ROWS / ways) + slot / ways;
+    const bool active = slot < ROWS && c < p.ncols;
+    const long long base = (static_cast<long long>(b) * p.Hkv + kvh) * p.max_splits;
+    const float *o_src = p.ws_o + (base * p.ncols + min(c, p.ncols - 1)) * D + 4 * e;
+    const float *ml_src = p.ws_ml + (base * p.ncols + min(c, p.ncols - 1)) * 2;
+    const long long step = static_cast<long long>(p.ncols);
+    float4_t o[kAhead];
+    float2_t ml[kAhead];
+    const auto load = [&](int s0) {
+#pragma unroll
+        for (int u = 0; u < kAhead; ++u) {
+            const int sp = min(s0 + u * ways, p.max_splits - 1);
+            ml[u] = *reinterpret_cast<const float2_u *>(ml_src + sp * step * 2);
+            o[u] = *reinterpret_cast<const float4_u *>(o_src + sp * step * D);
+        }
+    };
+    load(way);
     long long q_off;
     int L;
     seq_info(p, b, q_off, L);
     if (L <= 0 || L > p.rq) return;  // L > rq: written by fa_decode_kernel
     const int S = kv_len(p, b);
-    int nsplit = S <= 0 ? 1 : (S + p.split_len - 1) / p.split_len;
-    nsplit = min(nsplit, p.max_splits);
-    const long long base = (static_cast<long long>(b) * p.Hkv + kvh) * p.max_splits;
-    const int nc = p.ncols;
-    if (nsplit * nc <= kCombineStage) {
-        // all (m, l) pairs in one round of parallel loads
-        for (int i = threadIdx.x; i < nsplit * nc; i += blockDim.x) {
-            const float2 ml = *reinterpret_cast<const float2 *>(p.ws_ml + (base * nc + i) * 2);
-            wgt[i] = ml.x;
-            lsp[i] = ml.y;
+    const int nsplit = min(S <= 0 ? 1 : (S + p.split_len - 1) / p.split_len, p.max_splits);
+    float M = 0.0f, l = 0.0f;  // the maxima are clamped at 0
+    float4_t acc = {0.0f, 0.0f, 0.0f, 0.0f};
+    for (int s0 = way; s0 < nsplit; s0 += kAhead * ways) {
+        if (s0 != way) load(s0);
+        float Mn = M;
+#pragma unroll
+        for (int u = 0; u < kAhead; ++u)
+            if (s0 + u * ways < nsplit) Mn = fmaxf(Mn, ml[u].x);
+        const float f = __builtin_amdgcn_exp2f(M - Mn);
+        M = Mn;
+        l *= f;
+        acc *= f;
+#pragma unroll
+        for (int u = 0; u < kAhead; ++u)
+            if (s0 + u * ways < nsplit) {
+                const float g = __builtin_amdgcn_exp2f(ml[u].x - Mn);
+                l += g * ml[u].y;
+                acc += g * o[u];
+            }
+    }
+    if (ways > 1) {
+        if (slot < ROWS) {
+            acc_of[threadIdx.x] = acc;
+            if (e == 0) {
+                m_of[slot] = M;
+                l_of[slot] = l;
+            }
         }
         __syncthreads();
-        for (int c = threadIdx.x; c < nc; c += blockDim.x) {
-            float M = 0.0f;
-            for (int sp = 0; sp < nsplit; ++sp) M = fmaxf(M, wgt[sp * nc + c]);
-            float l = 0.0f;
-            for (int sp = 0; sp < nsplit; ++sp) {
-                const float f = __builtin_amdgcn_exp2f(wgt[sp * nc + c] - M);
-                wgt[sp * nc + c] = f;
-                l += f * lsp[sp * nc + c];
-            }
-            const float inv = l > 0.0f ? 1.0f / l : 0.0f;
-            for (int sp = 0; sp < nsplit; ++sp) wgt[sp * nc + c] *= inv;
+        if (!active || way != 0) return;
+        for (int w = 1; w < ways; ++w) M = fmaxf(M, m_of[slot + w]);
+        l = 0.0f;
+        acc = float4_t{0.0f, 0.0f, 0.0f, 0.0f};
+        for (int w = 0; w < ways; ++w) {
+            const float f = __builtin_amdgcn_exp2f(m_of[slot + w] - M);
+            l += f * l_of[slot + w];
+            acc += f * acc_of[threadIdx.x + w * V];
         }
-        __syncthreads();
-        for (int task = threadIdx.x; task < nc * D; task += blockDim.x) {
-            const int c = task / D, d = task % D;
-            const int hl = c / p.rq, row = c % p.rq;
-            if (hl >= p.G || row >= L) continue;
-            const float *src = p.ws_o + (base * nc + c) * D + d;
-            const long long step = static_cast<long long>(nc) * D;
-            float acc0 = 0.0f, acc1 = 0.0f, acc2 = 0.0f, acc3 = 0.0f;
-            int sp = 0;
-            for (; sp + 4 <= nsplit; sp += 4) {
-                acc0 += wgt[sp * nc + c] * src[sp * step];
-                acc1 += wgt[(sp + 1) * nc + c] * src[(sp + 1) * step];
-                acc2 += wgt[(sp + 2) * nc + c] * src[(sp + 2) * step];
-                acc3 += wgt[(sp + 3) * nc + c] * src[(sp + 3) * step];
-            }
-            for (; sp < nsplit; ++sp) acc0 += wgt[sp * nc + c] * src[sp * step];
-            const int h = kvh * p.G + hl;
-            p.o[((q_off + row) * p.H + h) * D + d] = Cvt<T>::from((acc0 + acc1) + (acc2 + acc3));
-        }
-        return;
     }
-    for (int task = threadIdx.x; task < nc * D; task += blockDim.x) {
-        const int c = task / D, d = task % D;
-        const int hl = c / p.rq, row = c % p.rq;
-        if (hl >= p.G || row >= L) continue;
-        float M = 0.0f;
-        for (int sp = 0; sp < nsplit; ++sp) M = fmaxf(M, p.ws_ml[((base + sp) * nc + c) * 2]);
-        float acc = 0.0f, l = 0.0f;
-        for (int sp = 0; sp < nsplit; ++sp) {
-            const float f = __builtin_amdgcn_exp2f(p.ws_ml[((base + sp) * nc + c) * 2] - M);
-            acc += f * p.ws_o[((base + sp) * nc + c) * D + d];
-            l += f * p.ws_ml[((base + sp) * nc + c) * 2 + 1];
-        }
-        const float out = l > 0.0f ? acc / l : 0.0f;
-        const int h = kvh * p.G + hl;
-        p.o[((q_off + row) * p.H + h) * D + d] = Cvt<T>::from(out);
-    }
+    const int hl = c / p.rq, row = c % p.rq;
+    if (!active || hl >= p.G || row >= L) return;
+    const float inv = l > 0.0f ? 1.0f / l : 0.0f;
+    store_row4<T>(p.o + ((q_off + row) * p.H + kvh * p.G + hl) * D + 4 * e, acc.x * inv, acc.y * inv,
+                  acc.z * inv, acc.w * inv);
 }
 
 // ------------------------------------------------------------------- host
@@ -541,13 +560,20 @@ Plan make_plan(int batch, int H, int Hkv, int q_hint, int k_hint) {
     // per slot of the 256 CUs, two each), with splits as long as that allows:
     // from 2048 keys down to 512.  Long splits write and merge fewer
     // partials; at B=64, Hkv=8 and kv_len <= 8192, 2048-key splits ran in
-    // 194 us against 217 us at 512.  Splits shorter than 512 keys cost more
-    // in per-workgroup start-up and merging than they gain in parallelism:
-    // one sequence of 32768 keys took 86 us with 128-key splits, 41 us with
-    // 512; 8 x 4096 keys 55 against 34 us.
+    // 194 us against 217 us at 512.
+    // Small grids go on down to one 128-key tile while all workgroups still
+    // run at once: then the time is a workgroup's serial chain of tiles.  32
+    // heads over 8, us at 512 / 256 / 128 keys: 1 x 600 16.4 / 12.4 / 11.0, 1 x
+    // 4096 18.0 / 13.9 / 12.1, 4 x 255..4095 19.1 / 14.7 / 12.8; over 1 kv head 1
+    // x 16384 18.8 / 15.2 / 14.6.  Past two workgroups per CU it turns: 4 of
+    // 255..700 keys by 32 kv heads 17.0 at 384 workgroups of 256, 22.3 at 768.
+    // Up to 512 keys are never split, so that such a call needs no scratch.
     const long long units = static_cast<long long>(batch) * Hkv;
+    const auto groups = [&](int len) { return units * ((k_hint + len - 1) / len); };
     int split = 2048;
-    while (split > 512 && units * ((k_hint + split - 1) / split) < 512) split >>= 1;
+    while (split > 512 && groups(split) < 512) split >>= 1;
+    if (k_hint > 512)
+        while (split <= 512 && split > kDecTile && groups(split / 2) <= 512) split >>= 1;
     pl.split_len = split;
     pl.max_splits = k_hint <= 0 ? 1 : (k_hint + split - 1) / split;
     return pl;
@@ -675,8 +701,13 @@ tecoopsStatus_t run(hipStream_t s, const FaParams &p, const Plan &pl) {
         hipLaunchKernelGGL(kern, grid, dim3(256), lds, s, p);
         TECO_CHECK_LAUNCH("flash_attention decode");
         if (pl.max_splits > 1) {
-            hipLaunchKernelGGL((fa_decode_combine_kernel<T, D>), dim3(p.batch * p.Hkv), dim3(256),
-                               0, s, p);
+            // as many ways as leave each kAhead splits or fewer
+            constexpr int rows = combine_rows<D>();
+            int ways = 1;
+            while (ways < rows && ways * kAhead < pl.max_splits) ways *= 2;
+            hipLaunchKernelGGL((fa_decode_combine_kernel<T, D>),
+                               dim3(p.batch * p.Hkv, tecoops::ceil_div(pl.ncols, rows / ways)), dim3(256),
+                               0, s, p, ways);
             TECO_CHECK_LAUNCH("flash_attention combine");
         }
         return TECOOPS_STATUS_SUCCESS;
@@ -878,6 +909,7 @@ tecoopsStatus_t fa_prepare(tecoopsHandle_t handle, int max_seqlen_q, int max_seq
         p.ncols = c.pl.ncols;
         p.split_len = c.pl.split_len;
         p.max_splits = c.pl.max_splits;
+        p.direct = static_cast<long long>(p.batch) * p.Hkv * p.max_splits <= tecoops::device_cus();
     } else {
         p.rq = 0x7fffffff;
     }
