@@ -100,4 +100,6 @@ def check(status, what=""):
 
 
 def call(name, *args):
-    check(getattr(lib(), name)(*args), name)
+    status = getattr(_LIB or lib(), name)(*args)
+    if status != SUCCESS:
+        raise TecoopsError(status, name)
