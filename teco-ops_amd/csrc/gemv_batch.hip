@@ -309,13 +309,17 @@ bool launch(const void *W, const void *sc, const void *x, void *y, int B, int N,
 // times).  fp16, batch 8, µs at 16 / 32 / 64 / 112 / 128 rows: [4096, 4096]
 // 7.9 / 9.2 / - / - / -, [6144, 4096] 11.9 / 10.2 / - / - / -, [14336, 4096]
 // - / 20.4 / 19.1 / - / -, [28672, 4096] - / 39.0 / 37.6 / 35.9 / 39.3; 8
-// against 16 rows [2048, 4096] 5.5 / 6.3.
-int rows_per_workgroup(int n, int least) {
+// against 16 rows [2048, 4096] 5.5 / 6.3.  For up to 8 rows of x (`few`, where
+// staging x costs least) 24, 48 and 56 fill in: with 24 against 8 [6144, 4096]
+// 10.3 / 12.5, 48 against 16 [11008, 4096] 15.5 / 18.0, 56 against 64 [14336,
+// 4096] 20.1 / 23.0 (weights rotated over 1 GB).
+int rows_per_workgroup(int n, int least, bool few) {
     const long long cus = tecoops::device_cus();
     int best = 128;
     long long best_load = -1;
-    for (int r : {128, 112, 96, 64, 32, 16, 8}) {
+    for (int r : {128, 112, 96, 64, 56, 48, 32, 24, 16, 8}) {
         if (r < least) break;
+        if (!few && (r == 56 || r == 48 || r == 24)) continue;
         const long long wgs = tecoops::ceil_div(n, r);
         const long long load = (wgs + cus - 1) / cus * r;
         if (best_load < 0 || load < best_load) {
@@ -332,7 +336,8 @@ int rows_per_workgroup(int n, int least) {
 // eight ways: fp16 21.0 / 20.0, int8 13.1 / 12.4 µs; int8 [4096, 4096], 2
 // stages a group: 5.5 / 6.3).  64 rows: two waves of 32 for 16-bit W (one
 // LDS read of x serves two row tiles), four of 16 for int8 ([14336, 4096]
-// batch 8: fp16 19.1 / 21.6, int8 13.6 / 12.3 µs).
+// batch 8: fp16 19.1 / 21.6, int8 13.6 / 12.3 µs).  24 and 56 rows: waves of 8
+// rows, since no 16-row waves divide them.
 template <typename T, bool I8, int XR>
 bool launch_rows(const void *W, const void *sc, const void *x, void *y, int B, int N, int K,
                  hipStream_t s) {
@@ -341,7 +346,7 @@ bool launch_rows(const void *W, const void *sc, const void *x, void *y, int B, i
     // faster than 32 ([4096, 14336] batch 64: 43.4 / 41.8 µs)
     constexpr bool kShortX = I8 && XR > 32;
     const int stages = (K / (I8 ? 16 : 8) + 15) / 16;
-    switch (rows_per_workgroup(N, kShortX ? 32 : 8)) {
+    switch (rows_per_workgroup(N, kShortX ? 32 : 8, XR <= 8)) {
         case 8:
             if constexpr (!kShortX) return launch<T, I8, XR, 8, 1, 4>(W, sc, x, y, B, N, K, s);
             return false;
@@ -350,7 +355,16 @@ bool launch_rows(const void *W, const void *sc, const void *x, void *y, int B, i
                 if (stages >= 32) return launch<T, I8, XR, 16, 1, 8>(W, sc, x, y, B, N, K, s);
             if constexpr (!kShortX) return launch<T, I8, XR, 16, 1, 4>(W, sc, x, y, B, N, K, s);
             return false;
+        case 24:
+            if constexpr (XR <= 8) return launch<T, I8, XR, 8, 3, 4>(W, sc, x, y, B, N, K, s);
+            return false;
         case 32: return launch<T, I8, XR, 16, 2, 2>(W, sc, x, y, B, N, K, s);
+        case 48:
+            if constexpr (XR <= 8) return launch<T, I8, XR, 16, 3, 2>(W, sc, x, y, B, N, K, s);
+            return false;
+        case 56:
+            if constexpr (XR <= 8) return launch<T, I8, XR, 8, 7, 2>(W, sc, x, y, B, N, K, s);
+            return false;
         case 64:
             if constexpr (I8)
                 return launch<T, I8, XR, 16, 4, (kShortX ? 1 : 2)>(W, sc, x, y, B, N, K, s);

@@ -138,7 +138,7 @@ class _DescSlots:
     argument, filled anew when the tensor's type, shape or strides differ from
     what the slot holds.  Creating, filling and freeing five of them took about
     half of a call's host time: a decode of 4 sequences of 255..4095 keys, whose
-    kernels take 11 us, had a host time of 16.6 us per call, now 7.0."""
+    kernels take 16 us, had a host time of 16.6 us per call, now 7.0."""
 
     def __init__(self, slots):
         self.d = [ctypes.c_void_p() for _ in range(slots)]

@@ -17,7 +17,10 @@ pytestmark = pytest.mark.gpu
 # N: 8, 16, 32, 64, 96, 112 and 128 rows per workgroup on 256 CUs
 SHAPES = [(3, 1, 8), (4, 2041, 136), (5, 2050, 520), (8, 4090, 72), (9, 6007, 200), (16, 301, 4104),
           (17, 11001, 120), (32, 3000, 1032), (33, 20001, 88), (48, 5003, 264), (49, 28003, 72),
-          (64, 32765, 40), (65, 1000, 392), (130, 60, 2056), (6, 28672, 256), (12, 32768, 128)]
+          (64, 32765, 40), (65, 1000, 392), (130, 60, 2056), (6, 28672, 256), (12, 32768, 128),
+          # up to 8 rows of x: 24, 48 and 56 rows, the last workgroup in part
+          (8, 6100, 1160), (3, 4097, 72), (5, 12001, 264), (8, 12288, 128), (8, 14335, 392),
+          (4, 12300, 520)]
 
 
 def _check(y, dt, ref, W, x, what):
