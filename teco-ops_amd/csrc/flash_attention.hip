@@ -657,6 +657,9 @@ bool prefill_wide(const FaParams &p, const Plan &pl) {
 //   Uneven batches (16..256 rows over 512..7936 cached keys each): 8 chunks 234
 //   / 98, 16 172 / 109, 32 267 / 161, 64 556 / 396; the hints hold only the
 //   longest, so the share is taken as about half of what they say.
+//   Where a cut in two would not fit the slots, contexts may yet be alike and
+//   the plan then cuts nothing, for 12 us (10 chunks of 91..307 rows over
+//   1954..3087 keys 104 / 116): only long contexts, for which that is little.
 //   Fresh prompts (nothing cached) have their tiles' lengths spread evenly
 //   and lose: 1 x 4096 157 / 180, 8 of 256..4096 95 / 108.
 // The 12-wave kernel reads K and V least often, the 4-wave one (a third of the
@@ -679,7 +682,8 @@ SplitArgs plan_split(const FaParams &p, const Plan &pl, int D) {
     const double tiles = static_cast<double>(p.Hkv) * (p.G / hw) * p.batch * std::ceil(mean / qt);
     const double share = tiles * (p.causal ? past + 0.5 * (mean + qt) : pl.rk) / slots;
     const bool uneven = pl.rq >= 1.5 * mean;
-    if (uneven ? pl.rk >= 0.8 * (0.55 * share + 800.0) : pl.rk >= (hw == 1 ? 2.0 : 1.5) * (share + 800.0))
+    if (pl.rk >= (hw == 1 ? 2.0 : 1.5) * (share + 800.0) ||
+        (uneven && pl.rk >= 0.8 * (0.55 * share + 800.0) && (2 * tiles <= slots || pl.rk >= 6144)))
         a.slots = slots;
     return a;
 }
