@@ -1011,8 +1011,11 @@ bool rows_aligned(const ConvArgs &a) {
 // 16.1 / 14.6, 8 x 85 14.4 / 13.4, 4 x 248 16.3 / 12.0, 64 x 10 22.1 / 15.7,
 // 64 x 40 43.5 / 27.1, 32 x 170 74.9 / 31.9, 32 x 274 112.5 / 53.1, 8 x 1950
 // 139.7 / 57.5; dim 1024, 64 x 10 8.1 / 8.7, 64 x 20 9.1 / 9.0, 64 x 39 13.6 /
-// 10.4.
+// 10.4.  And tokens from which it does: a wave takes groups of 512, so fewer
+// leave its lanes idle however many channels there are (dim 7360, 4 x 40 tokens,
+// width 2: 8.7 / 13.4).
 constexpr long long kAxisMinElems = 1 << 20;
+constexpr long long kAxisMinTokens = 512;
 
 template <int W, bool SILU>
 void launch(const ConvArgs &a0, bool seq_contig, long long max_len, hipStream_t s) {
@@ -1039,7 +1042,8 @@ void launch(const ConvArgs &a0, bool seq_contig, long long max_len, hipStream_t 
         return;
     }
     // (its waves read tokens that others' outputs would overwrite in place)
-    if (seq_contig && a.qsl != nullptr && a.x != a.out && max_len * a.dim >= kAxisMinElems) {
+    if (seq_contig && a.qsl != nullptr && a.x != a.out && max_len >= kAxisMinTokens &&
+        max_len * a.dim >= kAxisMinElems) {
         // groups of tokens of a channel, four at a time
         const long long groups = (max_len + 7 + kSegs * 512 - 1) / (kSegs * 512);
         const unsigned per_xcd = tecoops::ceil_div(a.dim, 8);
