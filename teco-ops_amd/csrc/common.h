@@ -10,7 +10,9 @@
 // wait is needed.  Each buffer grows on demand on the device current at the
 // op, and a slot taken over from another stream gets a new buffer; hipFree
 // synchronises the device first, so a buffer still read by enqueued work is
-// never freed or reused under it.
+// never freed or reused under it.  A request that can do without memory
+// (handle_scratch_if_any) never costs a buffer that is there: what it finds no
+// memory for it does not ask for again at every call.
 #pragma once
 
 #include <hip/hip_runtime.h>
@@ -23,6 +25,8 @@
 #include "tecoops.h"
 
 constexpr int kScratchSlots = 8;
+// Uses of a handle's scratch before a size that was refused is tried again.
+constexpr unsigned long long kScratchRetry = 1024;
 
 struct ScratchSlot {
     hipStream_t stream = nullptr;
@@ -35,6 +39,8 @@ struct tecoopsContext {
     hipStream_t stream = nullptr;
     ScratchSlot scratch[kScratchSlots];
     unsigned long long uses = 0;
+    size_t refused = 0;                // smallest optional size refused, 0: none
+    unsigned long long retry_at = 0;   // ... until this many uses
 };
 
 // Descriptor: same fields and stride rules as the reference
@@ -127,7 +133,8 @@ tecoopsStatus_t handle_scratch(tecoopsHandle_t handle, size_t bytes, void **out)
 
 // The same for an op that can do without: nullptr while the stream is
 // captured, when no memory is free, and when another stream would have to
-// give up its buffer.
+// give up its buffer.  The stream keeps the buffer it has unless a larger one
+// was allocated first.
 void *handle_scratch_if_any(tecoopsHandle_t handle, size_t bytes);
 
 }  // namespace tecoops

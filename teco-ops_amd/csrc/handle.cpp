@@ -236,13 +236,24 @@ bool stream_captured(hipStream_t stream) {
     return cs != hipStreamCaptureStatusNone;
 }
 
-// The buffer of the handle's current stream, of at least `bytes`; take_over:
-// from the least recently used stream if no slot is free.
-tecoopsStatus_t scratch_slot(tecoopsHandle_t handle, size_t bytes, bool take_over, void **out) {
-    if (bytes == 0) bytes = 256;
-    ScratchSlot *slot = nullptr;
+// The slot of the handle's current stream, or nullptr.
+ScratchSlot *own_slot(tecoopsHandle_t handle) {
     for (ScratchSlot &sl : handle->scratch)
-        if (sl.ptr != nullptr && sl.stream == handle->stream) slot = &sl;
+        if (sl.ptr != nullptr && sl.stream == handle->stream) return &sl;
+    return nullptr;
+}
+
+tecoopsStatus_t use_slot(tecoopsHandle_t handle, ScratchSlot *slot, void **out) {
+    slot->last_use = ++handle->uses;
+    *out = slot->ptr;
+    return TECOOPS_STATUS_SUCCESS;
+}
+
+// The buffer of the handle's current stream, of at least `bytes`, taken over
+// from the least recently used stream if no slot is free.
+tecoopsStatus_t scratch_slot(tecoopsHandle_t handle, size_t bytes, void **out) {
+    if (bytes == 0) bytes = 256;
+    ScratchSlot *slot = own_slot(handle);
     if (slot == nullptr) {  // a free slot, else the least recently used one
         slot = &handle->scratch[0];
         for (ScratchSlot &sl : handle->scratch) {
@@ -252,7 +263,6 @@ tecoopsStatus_t scratch_slot(tecoopsHandle_t handle, size_t bytes, bool take_ove
             }
             if (sl.last_use < slot->last_use) slot = &sl;
         }
-        if (slot->ptr != nullptr && !take_over) return TECOOPS_STATUS_ALLOC_FAILED;
         // A buffer taken over from another stream may still be read by work
         // enqueued there: free it (hipFree waits for the device) and let the
         // allocation below start afresh.
@@ -285,9 +295,39 @@ tecoopsStatus_t scratch_slot(tecoopsHandle_t handle, size_t bytes, bool take_ove
         slot->ptr = p;
         slot->bytes = grow;
     }
-    slot->last_use = ++handle->uses;
-    *out = slot->ptr;
-    return TECOOPS_STATUS_SUCCESS;
+    return use_slot(handle, slot, out);
+}
+
+// The same for an op that runs without it too: the new buffer is allocated
+// before the stream's old one is freed, so that a refusal changes nothing (an
+// op that needs the old one finds it), and a refused size is not asked for
+// again in the next kScratchRetry uses.  No slot is taken over.
+tecoopsStatus_t scratch_slot_if_any(tecoopsHandle_t handle, size_t bytes, void **out) {
+    ScratchSlot *slot = own_slot(handle);
+    if (slot != nullptr && slot->bytes >= bytes) return use_slot(handle, slot, out);
+    if (slot == nullptr) {
+        for (ScratchSlot &sl : handle->scratch)
+            if (sl.ptr == nullptr) {
+                slot = &sl;
+                break;
+            }
+        if (slot == nullptr) return TECOOPS_STATUS_ALLOC_FAILED;
+    }
+    if (handle->refused != 0 && bytes >= handle->refused && ++handle->uses < handle->retry_at)
+        return TECOOPS_STATUS_ALLOC_FAILED;
+    void *p = nullptr;
+    if (hipMalloc(&p, bytes) != hipSuccess) {
+        (void)hipGetLastError();
+        handle->refused = handle->refused == 0 || bytes < handle->refused ? bytes : handle->refused;
+        handle->retry_at = handle->uses + kScratchRetry;
+        return TECOOPS_STATUS_ALLOC_FAILED;
+    }
+    handle->refused = 0;
+    if (slot->ptr != nullptr && hipFree(slot->ptr) != hipSuccess) (void)hipGetLastError();
+    slot->stream = handle->stream;
+    slot->ptr = p;
+    slot->bytes = bytes;
+    return use_slot(handle, slot, out);
 }
 
 }  // namespace
@@ -303,7 +343,7 @@ tecoopsStatus_t handle_scratch(tecoopsHandle_t handle, size_t bytes, void **out)
                    "tecoopsFlashAttentionNoAlloc");
         return TECOOPS_STATUS_NOT_SUPPORTED;
     }
-    return scratch_slot(handle, bytes, true, out);
+    return scratch_slot(handle, bytes, out);
 }
 
 void *handle_scratch_if_any(tecoopsHandle_t handle, size_t bytes) {
@@ -317,7 +357,7 @@ void *handle_scratch_if_any(tecoopsHandle_t handle, size_t bytes) {
         (void)hipGetLastError();
         return nullptr;
     }
-    if (scratch_slot(handle, bytes, false, &out) != TECOOPS_STATUS_SUCCESS) out = nullptr;
+    if (scratch_slot_if_any(handle, bytes, &out) != TECOOPS_STATUS_SUCCESS) out = nullptr;
     if (hipThreadExchangeStreamCaptureMode(&mode) != hipSuccess) (void)hipGetLastError();
     return out;
 }
