@@ -144,8 +144,7 @@ __global__ void __launch_bounds__(256) fa_split_plan_kernel(FaParams p, SplitArg
         const int other = __builtin_amdgcn_readlane(key, v);
         rank += other > key || (other == key && v < lane) ? 1 : 0;
     }
-    part[0][rank] = lane;  // (every wave's sums in `part` have been read)
-    const int seq = part[0][lane];
+    const int seq = __builtin_amdgcn_ds_permute(rank << 2, lane);  // lane `rank` gets this lane's number
     const SeqPieces at = seq_pieces(p, seq, qt);
     // prefixes over the sequences in that order
     const int np = at.all(k), one = at.single(k);
