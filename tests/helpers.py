@@ -57,6 +57,31 @@ def assert_close(got, ref, atol=1e-2, rtol=1e-2, what=""):
     return err.max()
 
 
+def attention_row_bound(dtype):
+    """Largest distance of an attention output row (the D values of a token
+    and head) from the oracle's, relative to the row's 2-norm, on keys and
+    values drawn independently: the probabilities are rounded to 16 bits (u,
+    half a unit in the last place: at most u / sqrt(3) in the mean square, and
+    the terms p * v meet in the error with the signs they have in the row
+    itself) and so is the result: u * sqrt(2 / 3).  2 u allows for rows of few
+    or unluckily cancelling values; fp32 sums and merges add 1e-6."""
+    return 2 * (2.0 ** -11 if dtype == orc.HALF else 2.0 ** -8) + 1e-6
+
+
+def assert_rows_close(got, ref, dtype, what=""):
+    """Attention output against the oracle, row by row (attention_row_bound):
+    a tolerance that shrinks with the output, as an absolute one does not over
+    thousands of keys, so that a piece of the keys left out is seen."""
+    got, ref = np.asarray(got, np.float64), np.asarray(ref, np.float64)
+    err, norm = np.linalg.norm(got - ref, axis=-1), np.linalg.norm(ref, axis=-1)
+    bad = ~(err <= attention_row_bound(dtype) * norm)
+    if bad.any():
+        rel = np.where(norm > 0, err / np.maximum(norm, 1e-30), np.where(err > 0, np.inf, 0))
+        i = np.unravel_index(np.argmax(np.nan_to_num(rel, nan=np.inf)), rel.shape)
+        raise AssertionError(f"{what}: {bad.sum()} of {bad.size} rows out of tolerance; worst at {i}: "
+                             f"{rel[i]:.3e} of the row against {attention_row_bound(dtype):.3e}")
+
+
 def diff3_max(got, ref):
     """Reference harness criterion DIFF3_MAX (evaluator.h:62-63): max |d|/(|b|)
     where |b| >= 1e-4, else |d|.  Reported, not asserted."""
