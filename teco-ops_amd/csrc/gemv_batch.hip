@@ -169,8 +169,11 @@ gemv_batch_kernel(const char *__restrict__ W, const uint16_t *__restrict__ scale
         for (int t = 0; t < CT; ++t) acc[r][t] = f32x4_t{0.0f, 0.0f, 0.0f, 0.0f};
     // Workgroups start their sweep of K at different stages, so that the
     // requests in flight spread over the HBM channels (rows a power of two
-    // bytes apart start on the same one).
-    const int rot = (blockIdx.x * RS + (RS == 1 ? wave : 0)) % nst;
+    // bytes apart start on the same one).  The step is odd: nst mostly is a
+    // power of two, and an even step would leave most starts unused (bf16
+    // batch 8, steps of 2 / 3 stages: [16384, 8192] 81.0 / 47.6 µs, [32768,
+    // 4096] 44.3 / 42.8; steps of 8 / 9 at 128 rows [32768, 4096] 51.2 / 43.1).
+    const int rot = (blockIdx.x * (RS | 1) + (RS == 1 ? wave : 0)) % nst;
     char *wbuf = lds + wave * S::WB;
     char *xbuf = lds + NW * S::WB + kp * S::XB;
     const auto slot = [&](int i) { return __builtin_amdgcn_readfirstlane((i % D) * S::SB); };
