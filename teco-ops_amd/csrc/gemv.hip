@@ -6,11 +6,11 @@
 //   int8:         y[b, n] = fp16( s[n] * sum_k float(Wq[n, k]) * x[b, k] )
 //
 // gfx950 design, by batch size (rows of x):
-//   * 2-8 with int8 W of more than 32 rows per CU (4 or fewer rows of x, or
-//     up to 64 rows of W per CU) and K a multiple of 256: the 4x4x4
-//     matrix-core path ("4x4x4 MFMA path" below).  Each wave streams 4 whole
-//     rows of W in 256-byte row segments, x is copied into LDS straight from
-//     memory, and the waves start their sweeps of K at staggered offsets.
+//   * 2-8 with int8 W at the numbers of rows per CU in b8_takes() and K a
+//     multiple of 256: the 4x4x4 matrix-core path ("4x4x4 MFMA path" below).
+//     Each wave streams 4 whole rows of W in 256-byte row segments, x is copied
+//     into LDS straight from memory, and the waves start their sweeps of K at
+//     staggered offsets.
 //   * 3 and more (16-bit W), 2 and more (int8 W) otherwise, K in whole
 //     16-byte chunks of W: gemv_batch.hip, which copies W and x through LDS
 //     and streams W once for up to 64 rows of x.
@@ -544,17 +544,20 @@ constexpr int kRI8OneMaxK = 4096, kRI8OneMinN = 10240;
 // 15.9 and 16.3 us (two groups of 4 rows per wave: 15.0-15.6 us).
 constexpr int kB8CplI8 = 2, kB8MaxBatch = 8;
 
-// Whether the 4x4x4 path takes an int8 product: where it still beats
-// gemv_batch.hip, that is for more than 32 rows of W per CU up to batch 4, and
-// for 32 to 64 up to batch 8, with the staged x in LDS.  Batch 3 / 8, µs 4x4x4
-// and gemv_batch.hip: [14336, 4096] 11.5, 11.9 / 12.1, 12.3; [11008, 4096]
-// 10.0, 10.8 / 11.0, 11.6; [28672, 4096] 21.5, 21.4 / 25.7, 21.7; [22016,
-// 4096] 16.9, 17.5 / 19.8, 17.9; [8192, 4096] 9.1, 7.7 / 10.2, 8.1; [4096,
-// 14336] 12.6, 11.7 / 17.7, 12.4.
+// Whether the 4x4x4 path takes an int8 product, with the staged x in LDS: where
+// it still beats gemv_batch.hip.  Its waves are 4 rows each, so that its time
+// follows N closely, and up to batch 4 it reads x with half the LDS traffic.  µs
+// 4x4x4 / gemv_batch.hip at K = 4096: batch 4 [8192] 9.6 / 8.4, [9216] 9.9 /
+// 10.4, [14336] 12.3 / 12.7, [18432] 16.1 / 16.9, [21504] 17.7 / 17.9, [22528]
+// 19.0 / 18.5, [28672] 22.7 / 21.9, [34304] 27.1 / 28.8, [41984] 30.1 / 32.6,
+// [45056] 33.4 / 34.1, [57344] 39.1 / 40.2; batch 8 [12288] 12.0 / 11.8, [15360]
+// 13.5 / 14.1, [16384] 14.0 / 14.2, [17408] 20.8 / 17.0, [28672] 26.9 / 21.7.
 bool b8_takes(int batch, int n, int k) {
     const long long cus = tecoops::device_cus();
-    if (batch > kB8MaxBatch || k % 256 != 0 || n <= 32 * cus) return false;
-    if (batch > 4 && n > 64 * cus) return false;
+    if (batch > kB8MaxBatch || k % 256 != 0) return false;
+    if (batch <= 4 ? n <= 32 * cus || (n > 80 * cus && n <= 128 * cus)
+                   : n <= 48 * cus || n > 64 * cus)
+        return false;
     return (batch <= 4 ? 4 : 8) * 2LL * k <= kMaxLdsBytes;
 }
 

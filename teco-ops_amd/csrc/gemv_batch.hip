@@ -27,11 +27,13 @@
 // zero constant, for W and x alike, so any K in whole chunks works.
 #include "gemv_batch.h"
 
+#include "common.h"
 #include "device.h"
 
 namespace {
 
 using namespace tecoops::dev;
+using tecoops::gemv_batch_rows;
 
 typedef unsigned u32x4_t __attribute__((ext_vector_type(4)));
 typedef _Float16 f16x8_t __attribute__((ext_vector_type(8)));
@@ -307,40 +309,25 @@ bool launch(const void *W, const void *sc, const void *x, void *y, int B, int N,
     return true;
 }
 
-// Rows of W per workgroup: of the sizes built (8 .. 128), the one that leaves
-// the busiest CU the fewest rows, the largest on ties (it copies x the fewest
-// times).  fp16, batch 8, µs at 16 / 32 / 64 / 112 / 128 rows: [4096, 4096]
-// 7.9 / 9.2 / - / - / -, [6144, 4096] 11.9 / 10.2 / - / - / -, [14336, 4096]
-// - / 20.4 / 19.1 / - / -, [28672, 4096] - / 39.0 / 37.6 / 35.9 / 39.3; 8
-// against 16 rows [2048, 4096] 5.5 / 6.3.  For up to 8 rows of x (`few`, where
-// staging x costs least) 24, 48 and 56 fill in: with 24 against 8 [6144, 4096]
-// 10.3 / 12.5, 48 against 16 [11008, 4096] 15.5 / 18.0, 56 against 64 [14336,
-// 4096] 20.1 / 23.0 (weights rotated over 1 GB).
-int rows_per_workgroup(int n, int least, bool few) {
-    const long long cus = tecoops::device_cus();
-    int best = 128;
-    long long best_load = -1;
-    for (int r : {128, 112, 96, 64, 56, 48, 32, 24, 16, 8}) {
-        if (r < least) break;
-        if (!few && (r == 56 || r == 48 || r == 24)) continue;
-        const long long wgs = tecoops::ceil_div(n, r);
-        const long long load = (wgs + cus - 1) / cus * r;
-        if (best_load < 0 || load < best_load) {
-            best_load = load;
-            best = r;
-        }
-    }
-    return best;
-}
-
-// The waves of each size: K split over as many groups of waves as leave two
-// stages or more in LDS.  16 rows split K eight ways when that leaves
-// each group 4 stages or more and x is short ([4096, 14336] batch 8, four /
-// eight ways: fp16 21.0 / 20.0, int8 13.1 / 12.4 µs; int8 [4096, 4096], 2
-// stages a group: 5.5 / 6.3).  64 rows: two waves of 32 for 16-bit W (one
-// LDS read of x serves two row tiles), four of 16 for int8 ([14336, 4096]
-// batch 8: fp16 19.1 / 21.6, int8 13.6 / 12.3 µs).  24 and 56 rows: waves of 8
-// rows, since no 16-row waves divide them.
+// The waves of each size (gemv_batch_rows): K split over as many groups of
+// waves as leave two stages or more in LDS.  A wave's stages are a serial chain
+// of copies, LDS reads and MFMAs, so that where few rows leave a CU few waves,
+// more groups of shorter ranges are faster, as long as a group has enough
+// stages to run through:
+//   * 16 rows split K eight ways where that leaves each group 4 stages or more
+//     and x is short ([4096, 14336] batch 8, four / eight ways: fp16 21.0 /
+//     20.0, int8 13.1 / 12.4 µs; int8 [4096, 4096], 2 stages a group: 5.5 / 6.3);
+//   * 8 rows of int8 W with short x likewise, from 2 stages a group ([256,
+//     8192] batch 3, four / eight ways 7.0 / 6.0 µs, [1024, 13824] 10.7 / 8.5,
+//     [2048, 4096] 5.3 / 5.1);
+//   * 32 rows of int8 W with short x four ways where at most three quarters of
+//     the CUs have a workgroup ([5120, 13824] two / four ways: batch 3 19.1 /
+//     17.0, batch 8 20.2 / 18.1, [5120, 4096] 7.8 / 7.8, 8.1 / 7.6; two of the
+//     smaller workgroups share a CU, so full grids lose: [8192, 8192] batch 4
+//     14.1 / 15.9).
+// 64 rows: two waves of 32 for 16-bit W (one LDS read of x serves two row
+// tiles), four of 16 for int8 ([14336, 4096] batch 8: fp16 19.1 / 21.6, int8
+// 13.6 / 12.3 µs).
 template <typename T, bool I8, int XR>
 bool launch_rows(const void *W, const void *sc, const void *x, void *y, int B, int N, int K,
                  hipStream_t s) {
@@ -349,8 +336,11 @@ bool launch_rows(const void *W, const void *sc, const void *x, void *y, int B, i
     // faster than 32 ([4096, 14336] batch 64: 43.4 / 41.8 µs)
     constexpr bool kShortX = I8 && XR > 32;
     const int stages = (K / (I8 ? 16 : 8) + 15) / 16;
-    switch (rows_per_workgroup(N, kShortX ? 32 : 8, XR <= 8)) {
+    const int cus = tecoops::device_cus();
+    switch (gemv_batch_rows(N, K, B, I8, cus)) {
         case 8:
+            if constexpr (I8 && XR <= 8)
+                if (stages >= 16) return launch<T, I8, XR, 8, 1, 8>(W, sc, x, y, B, N, K, s);
             if constexpr (!kShortX) return launch<T, I8, XR, 8, 1, 4>(W, sc, x, y, B, N, K, s);
             return false;
         case 16:
@@ -358,15 +348,13 @@ bool launch_rows(const void *W, const void *sc, const void *x, void *y, int B, i
                 if (stages >= 32) return launch<T, I8, XR, 16, 1, 8>(W, sc, x, y, B, N, K, s);
             if constexpr (!kShortX) return launch<T, I8, XR, 16, 1, 4>(W, sc, x, y, B, N, K, s);
             return false;
-        case 24:
-            if constexpr (XR <= 8) return launch<T, I8, XR, 8, 3, 4>(W, sc, x, y, B, N, K, s);
-            return false;
-        case 32: return launch<T, I8, XR, 16, 2, 2>(W, sc, x, y, B, N, K, s);
+        case 32:
+            if constexpr (I8 && XR <= 8)
+                if (stages >= (XR <= 4 ? 32 : 16) && N <= 24 * cus)
+                    return launch<T, I8, XR, 16, 2, 4>(W, sc, x, y, B, N, K, s);
+            return launch<T, I8, XR, 16, 2, 2>(W, sc, x, y, B, N, K, s);
         case 48:
             if constexpr (XR <= 8) return launch<T, I8, XR, 16, 3, 2>(W, sc, x, y, B, N, K, s);
-            return false;
-        case 56:
-            if constexpr (XR <= 8) return launch<T, I8, XR, 8, 7, 2>(W, sc, x, y, B, N, K, s);
             return false;
         case 64:
             if constexpr (I8)

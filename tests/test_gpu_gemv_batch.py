@@ -1,8 +1,9 @@
 """Weight products of several rows of x (gemv_batch.hip), against the oracle,
 at the sizes where its tiling can go wrong: every number of W rows per
-workgroup (8 to 128, picked from N), the row remainders of each, every number
-of staged x rows (4 to 64) and the batches around it, slices of 64, K of one
-16-byte chunk, K that ends inside a stage, and K parts that are empty."""
+workgroup (8 to 128, picked from N and the batch), the row remainders of each,
+every number of staged x rows (4 to 64) and the batches around it, slices of
+64, K of one 16-byte chunk, K that ends inside a stage, and K parts that are
+empty."""
 import numpy as np
 import pytest
 import torch
@@ -14,11 +15,11 @@ from helpers import as_f32, bits, dev
 
 pytestmark = pytest.mark.gpu
 
-# N: 8, 16, 32, 64, 96, 112 and 128 rows per workgroup on 256 CUs
+# N: 8 to 128 rows per workgroup on 256 CUs
 SHAPES = [(3, 1, 8), (4, 2041, 136), (5, 2050, 520), (8, 4090, 72), (9, 6007, 200), (16, 301, 4104),
           (17, 11001, 120), (32, 3000, 1032), (33, 20001, 88), (48, 5003, 264), (49, 28003, 72),
           (64, 32765, 40), (65, 1000, 392), (130, 60, 2056), (6, 28672, 256), (12, 32768, 128),
-          # up to 8 rows of x: 24, 48 and 56 rows, the last workgroup in part
+          # up to 8 rows of x: 32, 48 and 64 rows, the last workgroup in part
           (8, 6100, 1160), (3, 4097, 72), (5, 12001, 264), (8, 12288, 128), (8, 14335, 392),
           (4, 12300, 520)]
 
@@ -57,6 +58,17 @@ def test_gemv_int8_batch(B, N, K):
     torch.cuda.synchronize()
     scaled = W.astype(np.float32) * orc.to_float(s)[:, None]
     _check(y, orc.HALF, orc.gemv_int8(W, s, x), scaled, orc.to_float(x), f"{B}x{N}x{K}")
+
+
+# int8 W with K split over more waves: 8 rows eight ways (from 16 stages of K),
+# 32 rows four ways (from 16, up to 4 rows of x 32, where few CUs have work),
+# with parts that end early or are empty, and the N and K just outside
+@pytest.mark.parametrize("B,N,K", [(2, 9, 4096), (3, 2047, 3856), (4, 2041, 3840), (5, 300, 4112),
+                                   (8, 2048, 13824), (7, 100, 7696), (2, 4104, 8192), (4, 5001, 7952),
+                                   (3, 6143, 13840), (4, 6145, 8192), (5, 5000, 3856), (8, 6000, 4096),
+                                   (6, 4999, 3840), (8, 4500, 12304), (4, 5000, 7936)])
+def test_gemv_int8_batch_split_k(B, N, K):
+    test_gemv_int8_batch(B, N, K)
 
 
 @pytest.mark.parametrize("N,K", [(40, 4104), (9000, 136)])
