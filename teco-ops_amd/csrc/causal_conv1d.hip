@@ -17,8 +17,9 @@
 //   token stride 1 (e.g. [batch, dim, seqlen], the reference's [dim, tokens]):
 //     a wave streams whole rows, lanes on consecutive 8-token chunks ->
 //     16-byte loads / stores, the W-1 overlap passed between lanes in
-//     registers (conv1d_rows_kernel); a varlen batch's channel is streamed
-//     across its sequences (conv1d_axis_kernel);
+//     registers (conv1d_rows_kernel); the channels of a varlen batch of short
+//     sequences are streamed across them (conv1d_axis_kernel, by the rule in
+//     causal_conv1d.h);
 //   channel stride 1 with dim % 8 == 0 (the reference C layout [tokens, dim]):
 //     a lane owns 8 consecutive channels (one 16-byte vector per token) of a
 //     16-token chunk of the global token axis; the W-1 rows before the chunk
@@ -29,6 +30,7 @@
 // state before writing the new one, so there is no cross-lane race
 // (conv1d_axis_kernel: one workgroup, with a barrier between the two).
 // HBM-bound: algorithmic bytes = 2 * (x + out) + weights + bias + state.
+#include "causal_conv1d.h"
 #include "common.h"
 #include "device.h"
 
@@ -246,36 +248,15 @@ __device__ __forceinline__ int line_misalign(const uint16_t *p) {
 // whole vectors are aligned wherever the row starts, as long as x and out are
 // off by the same amount (they are for equal strides); only the first and last
 // vectors of a row go element by element.  [8, 4096, 2051] 149.6 -> 58.4 us;
-// at [8, 4096, 1000], whose rows are aligned, it would take 35.0 against 30.3.
-//
-// Grid (channels / 4, sequences), 4 waves of one row each: at [8, 4096, 2048]
-// that is 32768 short-lived waves, which keep reads and writes of different
-// waves overlapped (47.5 us); 4 rows per wave made the resident waves load,
-// compute and store in lockstep (58.3 us).
+// at [8, 4096, 1000], whose rows are aligned, it would take 35.0 against 30.3,
+// so a row is asked where it starts.
 constexpr int kSegs = 4;
 
 template <int W, bool SILU, bool SHIFT>
-__global__ void __launch_bounds__(256) conv1d_rows_kernel(ConvArgs a) {
+__device__ __forceinline__ void conv1d_row(const ConvArgs &a, int b, int d, int cidx, long long len,
+                                           const uint16_t *xr, uint16_t *outr) {
     constexpr int CH = 8, SEG = 64 * CH;
     const int lane = threadIdx.x & 63;
-    const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
-    const int b = blockIdx.y, d = blockIdx.x * 4 + wave;
-    if (d >= a.dim) return;
-    long long len, xoff, ooff;
-    if (a.qsl != nullptr) {
-        const long long s0 = a.qsl[b];
-        len = a.qsl[b + 1] - s0;
-        xoff = s0 * a.xs;
-        ooff = s0 * a.os;
-    } else {
-        len = a.seq_len;
-        xoff = b * a.xb;
-        ooff = b * a.ob;
-    }
-    const int cidx = a.cidx ? a.cidx[b] : b;
-    if (cidx == a.pad_slot_id || len <= 0) return;
-    const uint16_t *xr = a.x + xoff + d * a.xd;
-    uint16_t *outr = a.out + ooff + d * a.od;
     const bool use_state =
         a.state != nullptr && (a.api_mode == 1 || (a.hinit != nullptr && a.hinit[b] != 0));
     uint16_t *st = a.state ? a.state + static_cast<long long>(cidx) * a.state_stride + d : nullptr;
@@ -354,6 +335,42 @@ __global__ void __launch_bounds__(256) conv1d_rows_kernel(ConvArgs a) {
 #pragma unroll
         for (int k = 0; k < W - 1; ++k) st[static_cast<long long>(k) * a.dim] = ns[k];
     }
+}
+
+// The row of sequence b and channel d (both wave-uniform).  ANY: it may start
+// anywhere, else both x and out are known to be on the boundary.
+template <int W, bool SILU, bool ANY>
+__device__ __forceinline__ void conv1d_row_at(const ConvArgs &a, int b, int d) {
+    long long len, xoff, ooff;
+    if (a.qsl != nullptr) {
+        const long long s0 = a.qsl[b];
+        len = a.qsl[b + 1] - s0;
+        xoff = s0 * a.xs;
+        ooff = s0 * a.os;
+    } else {
+        len = a.seq_len;
+        xoff = b * a.xb;
+        ooff = b * a.ob;
+    }
+    const int cidx = a.cidx ? a.cidx[b] : b;
+    if (cidx == a.pad_slot_id || len <= 0) return;
+    const uint16_t *xr = a.x + xoff + d * a.xd;
+    uint16_t *outr = a.out + ooff + d * a.od;
+    if (ANY && __builtin_amdgcn_readfirstlane(misalign(xr) | misalign(outr)) != 0)
+        conv1d_row<W, SILU, true>(a, b, d, cidx, len, xr, outr);
+    else
+        conv1d_row<W, SILU, false>(a, b, d, cidx, len, xr, outr);
+}
+
+// Grid (channels / 4, sequences), 4 waves of one row each: at [8, 4096, 2048]
+// that is 32768 short-lived waves, which keep reads and writes of different
+// waves overlapped (47.5 us); 4 rows per wave made the resident waves load,
+// compute and store in lockstep (58.3 us).
+template <int W, bool SILU, bool ANY>
+__global__ void __launch_bounds__(256) conv1d_rows_kernel(ConvArgs a) {
+    const int d = blockIdx.x * 4 + __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+    if (d >= a.dim) return;
+    conv1d_row_at<W, SILU, ANY>(a, blockIdx.y, d);
 }
 
 // ------------------------------------- ragged sequences along one token axis
@@ -484,7 +501,8 @@ __global__ void __launch_bounds__(256) conv1d_axis_kernel(ConvArgs a, int per_xc
         }
         // The tokens of this group that are among the first W-1 of their
         // sequence, over the values just stored (which have to be there
-        // first: another lane stored them).
+        // first: another lane stored them; a wave's stores to an address reach
+        // it in order, and the fence keeps the compiler to that).
         __builtin_amdgcn_fence(__ATOMIC_RELEASE, "workgroup");
         for (int base = b0; base < a.batch && q4[base] < g1; base += 64) {
             const int b = base + lane;
@@ -998,24 +1016,12 @@ bool tokens_layout(const ConvArgs &a) {
 // 18.3 / 15.7 us.  One token: 8 us against 134 us with one row per wave.
 constexpr long long kShortLenNear = 12, kShortLenFar = 4;
 
-// Every row of x and out starts on a 16-byte boundary.
+// Every row of x and out starts on a 16-byte boundary (with query_start_loc:
+// every channel's).
 bool rows_aligned(const ConvArgs &a) {
-    return a.qsl == nullptr && tecoops::aligned(a.x, 16) && tecoops::aligned(a.out, 16) &&
-           a.xd % 8 == 0 && a.xb % 8 == 0 && a.od % 8 == 0 && a.ob % 8 == 0;
+    return tecoops::aligned(a.x, 16) && tecoops::aligned(a.out, 16) && a.xd % 8 == 0 &&
+           a.od % 8 == 0 && (a.qsl != nullptr || (a.xb % 8 == 0 && a.ob % 8 == 0));
 }
-
-// Elements (tokens x channels) from which a varlen batch of token-contiguous
-// rows runs along the whole token axis (conv1d_axis_kernel), sequences short
-// enough for conv1d_short_kernel aside.  µs grouped or per-sequence rows /
-// token axis: dim 4096, 4 x 35 tokens 8.2 / 10.7, 8 x 16 8.6 / 11.0, 64 x 4.5
-// 16.1 / 14.6, 8 x 85 14.4 / 13.4, 4 x 248 16.3 / 12.0, 64 x 10 22.1 / 15.7,
-// 64 x 40 43.5 / 27.1, 32 x 170 74.9 / 31.9, 32 x 274 112.5 / 53.1, 8 x 1950
-// 139.7 / 57.5; dim 1024, 64 x 10 8.1 / 8.7, 64 x 20 9.1 / 9.0, 64 x 39 13.6 /
-// 10.4.  And tokens from which it does: a wave takes groups of 512, so fewer
-// leave its lanes idle however many channels there are (dim 7360, 4 x 40 tokens,
-// width 2: 8.7 / 13.4).
-constexpr long long kAxisMinElems = 1 << 20;
-constexpr long long kAxisMinTokens = 512;
 
 template <int W, bool SILU>
 void launch(const ConvArgs &a0, bool seq_contig, long long max_len, hipStream_t s) {
@@ -1041,11 +1047,12 @@ void launch(const ConvArgs &a0, bool seq_contig, long long max_len, hipStream_t 
         hipLaunchKernelGGL((conv1d_short_kernel<W, SILU>), dim3(grid), dim3(256), 0, s, a);
         return;
     }
-    // (its waves read tokens that others' outputs would overwrite in place)
-    if (seq_contig && a.qsl != nullptr && a.x != a.out && max_len >= kAxisMinTokens &&
-        max_len * a.dim >= kAxisMinElems) {
+    // (in place, the waves along the axis would read tokens that others' outputs
+    // overwrote)
+    if (seq_contig && a.qsl != nullptr && a.x != a.out &&
+        tecoops::conv1d_along_axis(a.batch, a.dim, max_len, tecoops::device_cus())) {
         // groups of tokens of a channel, four at a time
-        const long long groups = (max_len + 7 + kSegs * 512 - 1) / (kSegs * 512);
+        const long long groups = (max_len + 63 + kSegs * 512 - 1) / (kSegs * 512);
         const unsigned per_xcd = tecoops::ceil_div(a.dim, 8);
         hipLaunchKernelGGL((conv1d_axis_kernel<W, SILU>), dim3(8 * per_xcd),
                            dim3(64 * static_cast<unsigned>(groups < 4 ? groups : 4)), 0, s, a,
@@ -1070,7 +1077,7 @@ void launch(const ConvArgs &a0, bool seq_contig, long long max_len, hipStream_t 
     }
     if (seq_contig) {
         const dim3 grid(tecoops::ceil_div(a.dim, 4), a.batch);
-        if (rows_aligned(a))
+        if (a.qsl == nullptr && rows_aligned(a))
             hipLaunchKernelGGL((conv1d_rows_kernel<W, SILU, false>), grid, dim3(256), 0, s, a);
         else
             hipLaunchKernelGGL((conv1d_rows_kernel<W, SILU, true>), grid, dim3(256), 0, s, a);
