@@ -28,6 +28,7 @@ struct FaParams {
     float scale_log2;    // softmax_scale * log2(e)
     float inv_scale_log2;  // 1 / scale_log2: the rescale test compares raw scores
     int causal;
+    int turn;            // grid rows after which the sequences' places move on, as a shift
     long long total_q;   // rows of q and of the output (q's descriptor)
     // split-KV decode
     float *ws_o;         // [B][Hkv][max_splits][ncols][D]

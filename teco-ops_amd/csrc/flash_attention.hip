@@ -51,12 +51,15 @@
 #include <cstdio>
 
 #include "fa_device.h"
+#include "fa_grid.h"
 
 namespace {
 
 using tecoops::fa::FaCall;
 using tecoops::fa::Plan;
 using tecoops::fa::SplitArgs;
+using tecoops::fa::turn_shift;
+using tecoops::fa::turned_place;
 
 // A kernel's FaParams argument where it lies, at the start of the kernel
 // argument segment (constant address space): read through this pointer a
@@ -96,20 +99,6 @@ __device__ __attribute__((noinline)) void prefill_rest(const KernargParams *pp, 
 // W >= 12 asks for 3 waves per SIMD (168 VGPRs); head sizes above 128 with 4
 // waves one (their 4-wave tiles fill the registers), else 2.
 //
-// Sequence of grid column `col` (of batch) in grid row `row`.  Workgroup n runs
-// on XCD n % 8, and an XCD deals its workgroups to its 4 shader engines in
-// turn, each workgroup waiting for its own engine.  With a column fixed to a
-// sequence, a long sequence's workgroups (the only ones with work in the upper
-// rows) would keep to one engine of 4 when the columns repeat every 4: 3869 +
-// 3 x 1000 tokens, H32 Hkv8 D128 bf16, 358 us against 144 us for the 3869
-// alone.  The columns turn by one each row, each second row when the row
-// length itself alternates between two engines: 156 us; [2048, 3869, 720,
-// 1880] 359 -> 200, 8 x 256-2100 142 -> 94, 24 x 16-1024 48.6 -> 40.6 us,
-// equal lengths unchanged.
-__device__ __forceinline__ int turned_column(int col, int row, int batch) {
-    return (col + (row >> ((batch & 3) == 2))) % batch;
-}
-
 // The grid's tile rows are sized from max_seqlen_q, a bound the reference
 // never reads (flash_attention.cpp:98-99).  The workgroup of tile 0, which
 // is dispatched last, then takes every query tile past the grid in turn;
@@ -124,7 +113,7 @@ fa_prefill_kernel(FaParams p) {
     const int ngroups = p.G / HW;
     const int hg = blockIdx.x % ngroups;
     const int kvh = (blockIdx.x / ngroups) % p.Hkv;
-    const int b = turned_column(blockIdx.x / ngroups / p.Hkv, blockIdx.y, p.batch);
+    const int b = turned_place(blockIdx.x / ngroups / p.Hkv, blockIdx.y, p.turn, p.batch);
     const int rows = gridDim.y;  // tile rows sized from max_seqlen_q
     long long q_off;
     int L;
@@ -400,7 +389,7 @@ __global__ void __launch_bounds__(256, D > 128 ? 1 : 2) fa_decode_kernel(FaParam
         // do grids of no more workgroups than CUs, which all run at once (4
         // sequences of 255..4095 keys 12.8 / 11.0 us; up to two per CU even
         // lengths still gain 0.6, 8 uneven ones lose 2.5).
-        b = turned_column(blockIdx.x / p.Hkv, blockIdx.y, p.batch);
+        b = turned_place(blockIdx.x / p.Hkv, blockIdx.y, p.turn, p.batch);
         kvh = blockIdx.x % p.Hkv;
         split = blockIdx.y;
         seq_info(p, b, q_off, L);
@@ -588,7 +577,7 @@ size_t workspace_bytes(const Plan &pl, int batch, int Hkv, int D) {
 // Prefill over a grid of ceil(q_hint / QT) query tiles per (b, kv head, head
 // group); the workgroups of tile 0 cover any tiles past them.
 template <typename T, int D, int W, int HW, int QSUB, int BSM, int TILE>
-tecoopsStatus_t launch_prefill(const FaParams &p, const Plan &pl, hipStream_t s) {
+tecoopsStatus_t launch_prefill(FaParams p, const Plan &pl, hipStream_t s) {
     constexpr int QT = 32 * QSUB * (W / HW);
     auto *kern = &fa_prefill_kernel<T, D, W, HW, QSUB, BSM, TILE>;
     const size_t lds = prefill_lds_bytes<D, TILE, W, HW, QSUB, BSM>();
@@ -596,6 +585,7 @@ tecoopsStatus_t launch_prefill(const FaParams &p, const Plan &pl, hipStream_t s)
         return TECOOPS_STATUS_INTERNAL_ERROR;
     const int units = p.batch * p.Hkv * (p.G / HW);
     const int tiles = (pl.rq + QT - 1) / QT;
+    p.turn = turn_shift(p.Hkv * (p.G / HW), p.batch, pl.rq, p.total_q);
     hipLaunchKernelGGL(kern, dim3(units, tiles), dim3(W * 64), lds, s, p);
     TECO_CHECK_LAUNCH("flash_attention prefill");
     return TECOOPS_STATUS_SUCCESS;
@@ -913,6 +903,7 @@ tecoopsStatus_t fa_prepare(tecoopsHandle_t handle, int max_seqlen_q, int max_seq
         p.ncols = c.pl.ncols;
         p.split_len = c.pl.split_len;
         p.max_splits = c.pl.max_splits;
+        p.turn = turn_shift(p.Hkv, p.batch);
         p.direct = static_cast<long long>(p.batch) * p.Hkv * p.max_splits <= tecoops::device_cus();
     } else {
         p.rq = 0x7fffffff;
