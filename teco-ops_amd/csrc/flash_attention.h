@@ -79,6 +79,10 @@ tecoopsStatus_t prepare(tecoopsHandle_t handle, int max_seqlen_q, int max_seqlen
 // Bytes of split-KV partials the call needs (0 for prefill).
 size_t workspace_bytes(const FaCall &c);
 
+// The same from the sizes alone (H a multiple of Hkv), for a workspace of this
+// call's kv heads where tecoopsGetFlashAttentionWorkspaceSize covers any number.
+size_t workspace_bytes(int batch, int H, int Hkv, int D, int q_hint, int k_hint);
+
 // Bytes of partial states of a split prefill, and its launch (p.ws_o holds
 // them).
 size_t split_bytes(const SplitArgs &a, int D);

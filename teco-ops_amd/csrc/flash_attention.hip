@@ -957,6 +957,10 @@ tecoopsStatus_t prepare(tecoopsHandle_t handle, int max_seqlen_q, int max_seqlen
 
 size_t workspace_bytes(const FaCall &c) { return fa_workspace_bytes(c); }
 
+size_t workspace_bytes(int batch, int H, int Hkv, int D, int q_hint, int k_hint) {
+    return ::workspace_bytes(make_plan(batch, H, Hkv, q_hint, k_hint), batch, Hkv, D);
+}
+
 tecoopsStatus_t launch(hipStream_t s, FaCall &c, void *ws) { return fa_launch(s, c, ws); }
 
 }  // namespace fa
