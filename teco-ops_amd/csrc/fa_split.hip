@@ -11,7 +11,7 @@
 // result, depends on the lengths and the call's sizes alone.
 //
 // Bound like fa_prefill_kernel (a slot's serial loop over its keys); the plan
-// takes ~5 us, the merge 5-12.  16 chunks of 16..256 rows over 512..7936
+// takes ~6 us, the merge 5-14 (traced; 16 chunks as below 6.7 and 14.6).  16 chunks of 16..256 rows over 512..7936
 // cached keys (32 heads of 128 over 8 kv heads): 172 us unsplit, 109 split; 1 x
 // 32 rows over 16384 keys 432 / 42.  When a call is split: plan_split in
 // flash_attention.hip.

@@ -386,9 +386,10 @@ __global__ void __launch_bounds__(256, D > 128 ? 1 : 2) fa_decode_kernel(FaParam
         // Larger batches keep the grid's order, (sequence, kv head) by split:
         // with hundreds of items per CU the tail is short, and a scan over
         // every sequence in each workgroup would cost more than it saves.  So
-        // do grids of no more workgroups than CUs, which all run at once (4
-        // sequences of 255..4095 keys 12.8 / 11.0 us; up to two per CU even
-        // lengths still gain 0.6, 8 uneven ones lose 2.5).
+        // do grids of no more workgroups than CUs, which all run at once (32 heads
+        // over 8, us by the lookup / in grid order: 4 sequences of 255..1000 keys
+        // 13.1 / 11.5, 8 of 258..500 17.3 / 15.3, 1 x 4096 13.1 / 12.5; at up to two
+        // per CU 4 x 4095 20.8 / 20.1, but 8 of 258..1656 16.7 / 18.4).
         b = turned_place(blockIdx.x / p.Hkv, blockIdx.y, p.turn, p.batch);
         kvh = blockIdx.x % p.Hkv;
         split = blockIdx.y;
@@ -445,7 +446,7 @@ __global__ void __launch_bounds__(256, D > 128 ? 1 : 2) fa_decode_kernel(FaParam
 // ways splits the kernel is one trip to memory; the ways meet in LDS.  One
 // workgroup per (b, kv head), with the weights staged first and one thread per
 // element, took 4.4 us of 8 sequences of 255..4095 keys and 27 of 1 x 32768 by
-// 1 kv head (8 heads, 64 splits; the call 43 us, now 20).
+// 1 kv head (8 heads, 64 splits; the call 43 us, now 18).
 constexpr int kAhead = 4;
 
 template <int D>
@@ -552,10 +553,11 @@ Plan make_plan(int batch, int H, int Hkv, int q_hint, int k_hint) {
     // 194 us against 217 us at 512.
     // Small grids go on down to one 128-key tile while all workgroups still
     // run at once: then the time is a workgroup's serial chain of tiles.  32
-    // heads over 8, us at 512 / 256 / 128 keys: 1 x 600 16.4 / 12.4 / 11.0, 1 x
-    // 4096 18.0 / 13.9 / 12.1, 4 x 255..4095 19.1 / 14.7 / 12.8; over 1 kv head 1
-    // x 16384 18.8 / 15.2 / 14.6.  Past two workgroups per CU it turns: 4 of
-    // 255..700 keys by 32 kv heads 17.0 at 384 workgroups of 256, 22.3 at 768.
+    // heads over 8, us at 512 / 256 / 128 keys: 1 x 600 17.0 / 12.6 / 10.9, 1 x
+    // 4096 17.9 / 13.7 / 12.5, 4 of 255..1000 17.6 / 13.1 / 11.4; over 1 kv head 4
+    // x 4095 18.2 / 14.1 / 12.3.  Past two workgroups per CU it turns: 4 x 4095
+    // 21.1 / 20.8 / 27.1, 8 of 258..1656 18.2 / 16.7 / 23.2, 4 of 677..3209 18.4 /
+    // 15.8 / 16.1.
     // Up to 512 keys are never split, so that such a call needs no scratch.
     const long long units = static_cast<long long>(batch) * Hkv;
     const auto groups = [&](int len) { return units * ((k_hint + len - 1) / len); };
