@@ -227,7 +227,7 @@ tecoopsStatus_t tecoopsReshapeAndCacheEx(tecoopsHandle_t handle,
  * head size, max_seqlen_q and max_seqlen_k, and max_seqlen_k must then be > 0
  * (it sizes the split-KV partials).  A prefill without a workspace whose
  * longest context outweighs the rest (chunks of prompts over cached context)
- * splits its keys too, in up to 128 MiB of the handle's scratch per stream;
+ * splits its keys too, in up to 98 MiB of the handle's scratch per stream;
  * under capture, on more streams than the handle keeps scratch for, or where no
  * memory is free it runs unsplit, to the same results up to rounding. */
 tecoopsStatus_t tecoopsFlashAttentionEx(tecoopsHandle_t handle,

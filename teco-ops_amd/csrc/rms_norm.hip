@@ -39,8 +39,9 @@ __device__ __forceinline__ float block_sum(float v, float *red) {
 // asked for before the first use, the weight's too: with few rows the time is
 // one trip to memory, the reduction and the stores (8 x 4096 with residual:
 // 2.7 us, and a row of 512 takes 1.8; one wave per row waits for x, r
-// and w in turn over 8 chunks per lane, 8.8).
-template <typename T, int VPT, bool ADD>
+// and w in turn over 8 chunks per lane, 8.8).  STREAM: past the caches
+// (streams()).
+template <typename T, int VPT, bool ADD, bool STREAM>
 __global__ void __launch_bounds__(kRowThreads)
 rms_norm_row(const uint4 *__restrict__ x, const uint4 *__restrict__ w, const uint4 *__restrict__ r,
              uint4 *__restrict__ y, uint4 *__restrict__ r_out, int vec_per_row, int hidden,
@@ -53,8 +54,8 @@ rms_norm_row(const uint4 *__restrict__ x, const uint4 *__restrict__ w, const uin
         const int c = threadIdx.x + j * blockDim.x;
         v[j] = b[j] = wv[j] = uint4{0, 0, 0, 0};
         if (c < vec_per_row) {
-            v[j] = x[row + c];
-            if (ADD) b[j] = r[row + c];
+            v[j] = STREAM ? ld_stream(x + row + c) : x[row + c];
+            if (ADD) b[j] = STREAM ? ld_stream(r + row + c) : r[row + c];
             wv[j] = w[c];
         }
     }
@@ -89,8 +90,13 @@ rms_norm_row(const uint4 *__restrict__ x, const uint4 *__restrict__ w, const uin
             for (int q = 0; q < 4; ++q)
                 po[q] = pack<T>(lo<T>(pa[q]) * rstd * lo<T>(pw[q]),
                                 hi<T>(pa[q]) * rstd * hi<T>(pw[q]));
-            if (ADD) r_out[row + c] = v[j];
-            y[row + c] = o;
+            if constexpr (STREAM) {
+                if (ADD) st_stream(r_out + row + c, v[j]);
+                st_stream(y + row + c, o);
+            } else {
+                if (ADD) r_out[row + c] = v[j];
+                y[row + c] = o;
+            }
         }
     }
 }
@@ -197,11 +203,23 @@ void launch_wave(const void *x, const void *w, const void *r, void *y, void *ro,
                        static_cast<uint4 *>(ro), rows, hidden / 8, hidden, eps);
 }
 
+// Whether a workgroup per row reads and writes past the caches: where a call's
+// rows are half of the last one (256 MiB) and more, there is nothing to find there
+// but what they displace.  us, plain / streamed, in turn over 3 sets of buffers:
+// with residual 8192 x 4096 46.1 / 43.8, 4096 x 4096 24.6 / 23.4, 32768 x 2048 90.4 /
+// 84.8; smaller ones lose: 2048 x 5120 13.9 / 16.5.  Wider than 8192 it gains nothing.
+bool streams(long long rows, int hidden, bool add) {
+    return hidden <= 8192 && rows * hidden * (add ? 8 : 4) >= 128LL << 20;
+}
+
 template <typename T, int VPT, bool ADD>
 void launch_row(const void *x, const void *w, const void *r, void *y, void *ro, int rows, int hidden,
                 float eps, hipStream_t s) {
     const int nvec = hidden / 8, waves = (nvec + 64 * VPT - 1) / (64 * VPT);
-    hipLaunchKernelGGL((rms_norm_row<T, VPT, ADD>), dim3(rows), dim3(64 * waves), 0, s,
+    auto *kern = &rms_norm_row<T, VPT, ADD, false>;
+    if constexpr (VPT <= 2)
+        if (streams(rows, hidden, ADD)) kern = &rms_norm_row<T, VPT, ADD, true>;
+    hipLaunchKernelGGL(kern, dim3(rows), dim3(64 * waves), 0, s,
                        static_cast<const uint4 *>(x), static_cast<const uint4 *>(w),
                        static_cast<const uint4 *>(r), static_cast<uint4 *>(y),
                        static_cast<uint4 *>(ro), nvec, hidden, eps);
@@ -215,23 +233,30 @@ tecoopsStatus_t dispatch(tecoopsHandle_t handle, const void *x, const void *w, c
     for (const void *p : {x, w, r, static_cast<const void *>(y), static_cast<const void *>(ro)})
         if (p != nullptr) vec = vec && tecoops::aligned(p, 16);
     const int nvec = hidden / 8;
-    // Measured on bf16 rows, us, wave per row / workgroup per row: 8 rows of
-    // 4096 with residual 8.8 / 2.7, 8 of 1024 2.6 / 2.0, 1024 of 1024 3.4 / 3.1,
-    // 2048 of 1024 3.8 / 3.9, 1024 of 4096 7.3 / 5.6, 4096 of 4096 13.3 / 14.3,
-    // with residual 26.2 / 25.5, 4096 of 8192 29.5 / 22.6.  One chunk per lane
-    // (up to 512 wide) is the same trip to memory either way, and the wave has
-    // no barrier: 8 rows 2.0 / 2.0, 8192 rows 4.7 / 5.4.
-    const bool by_row = nvec > 512 || (nvec > 64 && (rows <= 1024 || (ADD && nvec >= 256)));
+    // us, wave per row / workgroup per row, in turn over 3 and over 8 sets of
+    // buffers: with residual 1000 x 2048 6.2 / 4.3, 6.4 / 4.9, 4096 x 2048 12.8 /
+    // 11.5, 13.2 / 14.1, 8192 x 4096 48.7 / 43.8, 49.6 / 44.4; without 1000 x 1024 2.7 /
+    // 2.6, 3.0 / 2.6, 2048 x 1024 3.2 / 3.2, 3.4 / 3.8, 1500 x 4096 5.6 / 6.6, 6.2 / 6.6,
+    // 4096 x 2048 5.9 / 7.6, 6.5 / 7.8; wider than 4096 1000 x 5120 5.9 / 5.7, 6.2 /
+    // 6.0, 2048 x 5120 7.7 / 9.0, 8.1 / 11.6, 4096 x 8192 22.6 / 24.4, 23.1 / 24.6, 8192 x
+    // 8192 50.2 / 45.6, 50.1 / 45.7.  One chunk per lane (up to 512 wide) is the same
+    // trip to memory either way, and the wave has no barrier: 8 rows 2.0 / 2.0, 8192
+    // rows 4.7 / 5.4.
+    const bool by_row = nvec > 64 && (rows <= 1024 || nvec > 1024 || (ADD && nvec >= 256) ||
+                                      (nvec > 512 && rows > 5120));
     if (vec && nvec <= 4 * kRowThreads && by_row) {
         if (nvec <= kRowThreads) launch_row<T, 1, ADD>(x, w, r, y, ro, rows, hidden, eps, s);
         else if (nvec <= 2 * kRowThreads) launch_row<T, 2, ADD>(x, w, r, y, ro, rows, hidden, eps, s);
         else launch_row<T, 4, ADD>(x, w, r, y, ro, rows, hidden, eps, s);
-    } else if (vec && nvec <= 64 * 8) {
+    } else if (vec && nvec <= 64 * 16) {
         const int vpt = (nvec + 63) / 64;
         if (vpt <= 1) launch_wave<T, 1, ADD>(x, w, r, y, ro, rows, hidden, eps, s);
         else if (vpt <= 2) launch_wave<T, 2, ADD>(x, w, r, y, ro, rows, hidden, eps, s);
         else if (vpt <= 4) launch_wave<T, 4, ADD>(x, w, r, y, ro, rows, hidden, eps, s);
-        else if constexpr (!ADD) launch_wave<T, 8, ADD>(x, w, r, y, ro, rows, hidden, eps, s);
+        else if constexpr (!ADD) {
+            if (vpt <= 8) launch_wave<T, 8, ADD>(x, w, r, y, ro, rows, hidden, eps, s);
+            else launch_wave<T, 16, ADD>(x, w, r, y, ro, rows, hidden, eps, s);
+        }
     } else {
         hipLaunchKernelGGL((rms_norm_scalar<T, ADD>), dim3(rows), dim3(kThreads), 0, s,
                            static_cast<const uint16_t *>(x), static_cast<const uint16_t *>(w),

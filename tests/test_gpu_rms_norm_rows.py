@@ -40,3 +40,30 @@ def test_rms_norm_rows(rows, D, residual, dt):
     assert ulp.max() <= 1
     if residual:
         assert np.array_equal(host_bits(rd), ref_sum)
+
+
+@pytest.mark.parametrize("dt", [orc.HALF, orc.BF16], ids=["fp16", "bf16"])
+@pytest.mark.parametrize("rows,D", [(1024, 4104), (1025, 4112), (1025, 8192), (1025, 8200), (5120, 4104),
+                                    (5121, 4104), (4096, 4096), (4095, 4096), (8192, 4096), (16400, 1024)])
+@pytest.mark.parametrize("residual", [False, True], ids=["pure", "add"])
+def test_rms_norm_many_rows(rows, D, residual, dt):
+    """A wave per row of 4104 to 8192 between 1025 and 5120 rows without residual,
+    past the caches from 128 MiB on, in place.  Units are counted on the number line:
+    the product of a zero, of which so many values hold some, rounds to fp16 with
+    either sign."""
+    r = np.random.default_rng(rows + D)
+    x, w = bits(r.standard_normal((rows, D)), dt), bits(r.uniform(0.5, 1.5, D), dt)
+    res = bits(r.standard_normal((rows, D)), dt) if residual else None
+    ref, ref_sum = orc.rms_norm(x, w, residual=res, eps=1e-6, dtype=dt)
+    xd, wd = dev(x, dt), dev(w, dt)
+    rd = dev(res, dt) if residual else None
+    tecoops.rms_norm(xd, wd, rd, xd, rd, 1e-6)
+    torch.cuda.synchronize()
+
+    def line(v):
+        v = v.astype(np.int32)
+        return np.where(v & 0x8000, -(v & 0x7fff), v)
+
+    assert np.abs(line(host_bits(xd)) - line(ref)).max() <= 1
+    if residual:
+        assert np.array_equal(host_bits(rd), ref_sum)
