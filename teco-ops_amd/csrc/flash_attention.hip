@@ -648,7 +648,10 @@ bool prefill_wide(const FaParams &p, const Plan &pl) {
 //   per kv head: its tiles are 384 rows).
 //   Uneven batches (16..256 rows over 512..7936 cached keys each): 8 chunks 234
 //   / 98, 16 172 / 109, 32 267 / 161, 64 556 / 396; the hints hold only the
-//   longest, so the share is taken as about half of what they say.
+//   longest, so the share is taken as about half of what they say.  Below some
+//   1200 keys past it the gain is down to what the plan and merge take: 40 heads
+//   over 8, 9 chunks of 5..21 rows over 919..1272 keys 47 / 56; 32 over 8, 4 of 95..460
+//   over 481..520 27 / 34, 6 of 9..238 over 679..1454 49 / 45.
 //   Where a cut in two would not fit the slots, contexts may yet be alike and
 //   the plan then cuts nothing, for 12 us (10 chunks of 91..307 rows over
 //   1954..3087 keys 104 / 116): only long contexts, for which that is little.
@@ -675,7 +678,7 @@ SplitArgs plan_split(const FaParams &p, const Plan &pl, int D) {
     const double share = tiles * (p.causal ? past + 0.5 * (mean + qt) : pl.rk) / slots;
     const bool uneven = pl.rq >= 1.5 * mean;
     if (pl.rk >= (hw == 1 ? 2.0 : 1.5) * (share + 800.0) ||
-        (uneven && pl.rk >= 0.8 * (0.55 * share + 800.0) && (2 * tiles <= slots || pl.rk >= 6144)))
+        (uneven && pl.rk >= 0.44 * share + 1200.0 && (2 * tiles <= slots || pl.rk >= 6144)))
         a.slots = slots;
     return a;
 }
