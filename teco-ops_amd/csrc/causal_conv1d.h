@@ -5,13 +5,19 @@
 namespace tecoops {
 
 // Whether a varlen batch of token-contiguous rows runs along the token axis
-// (conv1d_axis_kernel): where that is ahead of a wave per sequence and channel
-// (or its grouped form) on ragged batches and no slower on batches whose
-// sequences all start on the 16-byte boundary, which the host cannot tell apart.
-// Its workgroup per channel takes at most 4 groups of 2048 tokens at a time, so
-// that it wants channels to fill the chip, and pays where the sequences are
-// short against a group.  µs by rows / along the axis on 256 CUs, sequences on
-// the boundary, then off it or of random length:
+// (conv1d_axis_kernel) or a wave per sequence and channel (or its grouped form).
+// Along the axis a workgroup per channel takes at most 4 groups of 2048 tokens at a
+// time, so that it wants channels to fill the chip, and pays where the sequences
+// are short against a group, and where they start off the 16-byte boundary, which
+// costs a wave per row more.  The host knows their total only: lengths that are
+// alike and whole vectors leave one that 8 times their number divides, which other
+// lengths hardly ever do.
+// Not divided: µs by rows / along the axis on 256 CUs: 44 sequences of 12..23
+// tokens, dim 6336 32 / 18; 100 of 9 in the mean, 6360 53 / 23; 26 of 32, 4840 26 /
+// 14; 7 of 163, 2704 16 / 9; 6 of 637, 6544 44 / 28; 20 of 1186, 1192 41 / 28; but 7 of
+// 62, 4520 11 / 12, and few channels of long ones: 54 of 1106, 272 26 / 36.
+// Divided: µs by rows / along the axis, sequences on the boundary, then off it or
+// of random length:
 //   mean length to 256: dim 512, 64 x 256 18.5 / 15.4, 25.9 / 20.1; dim 384,
 //     64 x 256 14.8 / 15.4, 21.7 / 19.1, 512 x 40 29 / 27, 39 / 27; dim 256
 //     19.3 / 20.1, 24.8 / 21.1; dim 64, 64 x 256 6.5 / 9.8
@@ -28,8 +34,14 @@ namespace tecoops {
 // wave each: dim 1024, 1 x 16384 23.5 / 17.1, 25.8 / 21.5; dim 64 20.8 / 8.0;
 // dim 2048 30.4 / 34.9; dim 768, 2 x 4096 10.8 / 8.9, 12.7 / 13.7, 3001 + 900
 // tokens 9.9 / 8.2.
+// Over 1000 random batches (1..128 sequences, 64..8192 channels, a third alike) the
+// choice takes 1.6 % more than the better kernel in the mean.
 inline bool conv1d_along_axis(long long batch, long long dim, long long tokens, long long cus) {
     if (batch <= 2 && tokens >= 3072 && batch * dim <= 6 * cus) return true;
+    if (tokens % (8 * batch) != 0) {
+        if (tokens * dim < (1LL << 20) || dim < cus || tokens > batch * (dim >= 3 * cus ? 2048 : 512)) return false;
+        return (tokens >= 448 && batch * dim >= 96 * cus) || (tokens >= 1024 && batch * dim >= 16 * cus);
+    }
     if (tokens < 1024 || (tokens < 2048 && tokens * dim < (1LL << 22))) return false;
     const long long mean = (tokens + batch - 1) / batch;
     if (mean <= 256) return 2 * dim >= 3 * cus;

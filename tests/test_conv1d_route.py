@@ -48,3 +48,14 @@ def test_what_gains_runs_along_the_axis(along_axis):
     for batch, dim, tokens in ((16, 4096, 8064), (64, 512, 64 * 256), (512, 4096, 512 * 40), (32, 1024, 29561),
                                (1, 64, 16384), (2, 768, 3901), (32, 2048, 2140)):
         assert along_axis(batch, dim, tokens)
+
+
+def test_ragged_batches_run_along_the_axis(along_axis):
+    """Lengths that are not alike in whole vectors, by their total: many short
+    sequences, and longer ones of many channels; not a few tokens, nor few channels
+    of long sequences."""
+    for batch, dim, tokens in ((44, 6336, 750), (100, 6360, 873), (26, 4840, 831), (7, 2704, 1142), (6, 6544, 3821),
+                               (20, 1192, 23715), (52, 360, 14260)):
+        assert along_axis(batch, dim, tokens)
+    for batch, dim, tokens in ((7, 4520, 434), (8, 4888, 512), (54, 272, 59702), (5, 736, 44727), (99, 216, 17744)):
+        assert not along_axis(batch, dim, tokens)
